@@ -17,8 +17,10 @@
 // rows of Wt, 8 contiguous k) and W [K][nout] (backward data: 8 contiguous
 // output columns).
 #include <hip/hip_runtime.h>
+#include <climits>
 #include <cstdint>
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/cabanadem_gnn.h"
 
@@ -1117,6 +1119,8 @@ __global__ __launch_bounds__(kThreads) void k_bcast_add(const float* d_agg, cons
   for (int q = 0; q < 8; ++q) dst[q] += src[q];
 }
 
+#include "gnn_train_kernels.h"
+
 // Adam on a flat FP32 parameter vector (bias-corrected step sizes precomputed).
 __global__ __launch_bounds__(kThreads) void k_adam(float* p, const float* g, float* m, float* v, long n,
                                                    float lr_t, float b1, float b2, float eps,
@@ -1601,6 +1605,23 @@ int launch_edge(const EdgeFwdArgs& a, int grid_cap, void* stream) {
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
+// Rows of a chunk of the parameter gradients, at least.
+#ifndef GNN_GRAD_ROWS
+#define GNN_GRAD_ROWS 512
+#endif
+constexpr int kGradRows = GNN_GRAD_ROWS;
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+template <int NO>
+int launch_bwd_rows(const BwdRowsArgs& a, int nx, int grid, hipStream_t s) {
+  const dim3 g(grid), b(64 * kBwdWaves);
+  if (nx == 0) hipLaunchKernelGGL((k_bwd_rows<NO, 0>), g, b, 0, s, a);
+  else if (nx == 1) hipLaunchKernelGGL((k_bwd_rows<NO, 1>), g, b, 0, s, a);
+  else hipLaunchKernelGGL((k_bwd_rows<NO, 2>), g, b, 0, s, a);
+  return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
 bool edge_weights_ok(const gnn_mlp_weights* wt) {
   return wt && wt->K == 3 * kLat && wt->nout == kLat && wt->nout_pad == kLat && wt->W1t && wt->W2t && wt->b1 &&
          wt->b2;
@@ -1696,6 +1717,99 @@ int gnn_weight_grad(const gnn_mlp_io* io, const void* G_bf16, const float* G_f32
   hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(cw)), dim3(kThreads), 0, s, part, nch, cw, dW, accumulate);
   hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(a.NC)), dim3(kThreads), 0, s, bpart, nch, (long)a.NC, db,
                      accumulate);
+  return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+int gnn_mlp_grads(const gnn_mlp_io* io, const gnn_mlp_weights* wt, const float* dY, const float* add,
+                  const int* add_idx, const void* hidden, float* const dX[3], int accumulate, void* dH,
+                  void* dYb, float* work, long work_floats, float* grad, void* stream) {
+  if (check_io(io) || !wt || (!dY && !add) || (add && !add_idx) || !hidden || !dH || !dYb || !work || !grad ||
+      !wt->W1 || !wt->W2)
+    return -1;
+  const bool wide = wt->nout_pad == kLat && wt->nout == kLat;
+  if (!wide && (wt->nout_pad != 16 || wt->nout < 1 || wt->nout > 16 || add || !dY)) return -1;
+  const Segs in = make_segs(io);
+  const int K = in.start[io->nseg];
+  const bool narrow = io->nseg == 1 && io->width[0] == 32;
+  if (K != wt->K) return -1;
+  for (int q = 0; q < io->nseg; ++q)
+    if ((io->width[q] != kLat && !narrow) || !aligned16(io->src[q])) return -1;
+  if (!aligned16(dY) && wide) return -1;
+  if (!aligned16(add) || !aligned16(hidden) || !aligned16(dH) || !aligned16(dYb) || !aligned16(work) ||
+      !aligned16(grad))
+    return -1;
+  const int cus = device_cus();
+  if (cus <= 0) return -2;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  BwdRowsArgs a{};
+  a.M = io->M;
+  a.nout = wt->nout;
+  a.dY = dY;
+  a.add = add;
+  a.idx = add_idx;
+  a.hid = reinterpret_cast<const bf16*>(hidden);
+  a.W2 = reinterpret_cast<const bf16*>(wt->W2);
+  a.dH = reinterpret_cast<bf16*>(dH);
+  a.dYb = reinterpret_cast<bf16*>(dYb);
+  int nx = 0;
+  for (int q = 0; dX && q < io->nseg; ++q) {
+    if (!dX[q]) continue;
+    if (nx == 2 || narrow || !aligned16(dX[q])) return -1;
+    a.W1[nx] = reinterpret_cast<const bf16*>(wt->W1) + (long)in.start[q] * kLat;
+    a.dX[nx] = dX[q];
+    // dY of the same rows is in registers when its gradient accumulates there
+    const bool acc = (accumulate >> q) & 1;
+    a.mode[nx] = !acc ? 0 : (wide && (dX[q] == dY || !dY) ? 2 : 1);
+    ++nx;
+  }
+  const long cw = (long)(K + 1) * kLat + (long)kLat * wt->nout_pad;
+  const int per = 16 * kBwdWaves;
+  int grid = (io->M + per - 1) / per;
+  if (grid > cus) grid = cus;
+  // chunks of the parameter gradients: one block per CU over all 128-wide
+  // blocks of columns, chunks a multiple of 8 (the blocks of one chunk then
+  // share an XCD's L2) and at least kGradRows rows each
+  const int nby = (narrow ? 1 : io->nseg) + 1;
+  int nch = cus / nby / 8 * 8;
+  const int most = (io->M + kGradRows - 1) / kGradRows;
+  if (nch < 1) nch = 1;
+  if (nch > most) nch = most;
+  const int step = 32 * kWgWaves;
+  const int chunk = ((io->M + nch - 1) / nch + step - 1) / step * step;
+  nch = (io->M + chunk - 1) / chunk;
+  if ((long)grid * kBiasCols + (long)nch * cw > work_floats) return -1;
+  a.bpart = work;
+  if (int r = wide ? launch_bwd_rows<kLat>(a, nx, grid, s) : launch_bwd_rows<16>(a, nx, grid, s)) return r;
+  WgradPairArgs g{};
+  g.M = io->M;
+  g.K = K;
+  g.NO = wt->nout_pad;
+  g.chunk = chunk;
+  g.in = in;
+  g.dH = a.dH;
+  g.hid = a.hid;
+  g.dYb = a.dYb;
+  g.part = work + (long)grid * kBiasCols;
+  const dim3 gg(nch, nby), gb(64 * kWgWaves);
+  if (narrow && wide) hipLaunchKernelGGL((k_wgrad_pair<2, 8>), gg, gb, 0, s, g);
+  else if (narrow) hipLaunchKernelGGL((k_wgrad_pair<2, 1>), gg, gb, 0, s, g);
+  else if (wide) hipLaunchKernelGGL((k_wgrad_pair<8, 8>), gg, gb, 0, s, g);
+  else hipLaunchKernelGGL((k_wgrad_pair<8, 1>), gg, gb, 0, s, g);
+  hipLaunchKernelGGL(k_grad_reduce, dim3((unsigned)(cw / kLat + 1)), dim3(kThreads), 0, s, (const float*)g.part, nch,
+                     (const float*)a.bpart, grid, K, wt->nout_pad, grad);
+  return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+int gnn_edge_hidden_grad_to_nodes(int N, const void* dH, const int* row, const int* rev,
+                                  const gnn_mlp_weights* wt, float* dh, void* stream) {
+  if (N <= 0 || !dH || !row || !rev || !dh || !edge_weights_ok(wt) || !wt->W1 || !aligned16(dH) || !aligned16(dh))
+    return -1;
+  const int cus = device_cus();
+  if (cus <= 0) return -2;
+  EdgeToNodesArgs a{N, reinterpret_cast<const bf16*>(dH), row, rev, reinterpret_cast<const bf16*>(wt->W1), dh};
+  const int blocks = (N + 16 * kToNodesWaves - 1) / (16 * kToNodesWaves);
+  hipLaunchKernelGGL(k_edge_hidden_to_nodes, dim3(blocks < cus ? blocks : cus), dim3(64 * kToNodesWaves), 0,
+                     reinterpret_cast<hipStream_t>(stream), a);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

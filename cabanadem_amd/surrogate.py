@@ -38,6 +38,7 @@ LAT = 128
 FEAT = 32
 HIST = 5
 GNN_ABI_VERSION = 5
+GRAD_WORK_FLOATS = 5 << 20  # include/cabanadem_gnn.h GNN_GRAD_WORK_FLOATS
 
 _vp = C.c_void_p
 _ip = C.POINTER(C.c_int)
@@ -63,6 +64,9 @@ _SIG = {
                                    C.POINTER(_vp), C.c_int, C.c_int, _vp]),
     "gnn_weight_grad": (C.c_int, [C.POINTER(GnnMlpIo), _vp, _vp, C.c_int, C.c_int, _vp, _vp, C.c_int,
                                   _vp, _vp, C.c_int, _vp]),
+    "gnn_mlp_grads": (C.c_int, [C.POINTER(GnnMlpIo), C.POINTER(GnnMlpWeights), _vp, _vp, _vp, _vp,
+                                C.POINTER(_vp), C.c_int, _vp, _vp, _vp, C.c_long, _vp, _vp]),
+    "gnn_edge_hidden_grad_to_nodes": (C.c_int, [C.c_int, _vp, _vp, _vp, C.POINTER(GnnMlpWeights), _vp, _vp]),
     "gnn_segment_sum": (C.c_int, [_vp, _vp, C.c_int, _vp, _vp]),
     "gnn_edge_grad_to_nodes": (C.c_int, [_vp, _vp, _vp, _vp, C.c_int, _vp, _vp]),
     "gnn_broadcast_add": (C.c_int, [_vp, _vp, C.c_long, _vp, _vp]),
@@ -316,8 +320,7 @@ class Network:
         self.cast()
         self.cap_N = self.cap_E = 0
         self.h = self.e = None
-        self.part = self.bpart = None
-        self.nchunks = 64
+        self.work = None
 
     # -- parameters --------------------------------------------------------
     def cast(self):
@@ -352,11 +355,11 @@ class Network:
         hidden layers and the gradient buffers exist only once the network
         has trained."""
         torch = _torch()
-        first_train = train and self.part is None
+        first_train = train and self.work is None
         grow_n, grow_e = N > self.cap_N or self.h is None, E > self.cap_E or self.e is None
         if not (grow_n or grow_e or first_train):
             return
-        train = train or self.part is not None
+        train = train or self.work is not None
         bf, f32, dev = torch.bfloat16, torch.float32, self.dev
         L = self.L
         z = lambda *s, dt=bf: torch.zeros(s, dtype=dt, device=dev)
@@ -374,6 +377,7 @@ class Network:
                 self.d_h = z(N, LAT, dt=f32)
                 self.d_agg = z(N, LAT, dt=f32)
                 self.dH_n = z(N, LAT)
+                self.dY_n = z(N, LAT)
         if grow_e or first_train:
             E = max(E * 5 // 4, self.cap_E) if grow_e else self.cap_E
             self.cap_E = E
@@ -382,12 +386,10 @@ class Network:
             self.hid_enc_e = z(E, LAT) if train else None
             if train:
                 self.d_e = z(E, LAT, dt=f32)
-                self.d_hi = z(E, LAT, dt=f32)
-                self.d_hj = z(E, LAT, dt=f32)
                 self.dH_e = z(E, LAT)
-        if train and self.part is None:
-            self.part = z(self.nchunks * 3 * LAT * LAT, dt=f32)
-            self.bpart = z(self.nchunks * LAT, dt=f32)
+                self.dY_e = z(E, LAT)
+        if train and self.work is None:
+            self.work = torch.empty(GRAD_WORK_FLOATS, dtype=f32, device=dev)
 
     # -- forward -----------------------------------------------------------
     def _fwd(self, mlp, inp, res, hid, out, outf, train):
@@ -462,86 +464,49 @@ class Network:
         return self.out[:N]
 
     # -- backward ----------------------------------------------------------
-    def _wgrad(self, mlp, inp, hid, dH, dY32, M, accumulate=0):
-        Lb, s = glib(), stream()
-        base = self.grad.data_ptr()
-        # W2, b2: X = hidden, G = dY (float [M][nout])
-        _ok(Lb.gnn_weight_grad(C.byref(io(M, (hid, None))), None, ptr(dY32), mlp.nout, mlp.NP,
-                               ptr(self.part), ptr(self.bpart), self.nchunks,
-                               C.c_void_p(base + 4 * mlp.o_W2), C.c_void_p(base + 4 * mlp.o_b2),
-                               accumulate, s), "wgrad W2")
-        # W1, b1: X = the MLP input, G = dH (bf16 [M][128])
-        _ok(Lb.gnn_weight_grad(C.byref(inp), ptr(dH), None, LAT, LAT, ptr(self.part), ptr(self.bpart),
-                               self.nchunks, C.c_void_p(base + 4 * mlp.o_W1),
-                               C.c_void_p(base + 4 * mlp.o_b1), accumulate, s), "wgrad W1")
-
     def backward(self, g: Graph, xn, xe, d_out):
         """d_out float [N][3]: gradient of the loss at the decoder output.
         Fills self.grad (overwritten)."""
-        torch = _torch()
         Lb, s, N, E = glib(), stream(), g.N, g.E
         F = self.flat
-        bwd = lambda mlp, inp, dY, hid, dH, dX, acc, M: _ok(
-            Lb.gnn_mlp_backward(C.byref(inp), C.byref(mlp.weights(F)), ptr(dY), ptr(hid), ptr(dH),
-                                (C.c_void_p * 3)(*[None if d is None else d.data_ptr() for d in dX]),
-                                acc, 0, s), "mlp backward")
-        d_h = self.d_h[:N]
-        # decoder
-        inp = io(N, (self.h[self.L][:N], None))
-        dH = self.dH_n[:N]
-        bwd(self.dec, inp, d_out, self.hid_dec, dH, [d_h, None, None], 0, N)
-        self._wgrad(self.dec, inp, self.hid_dec, dH, d_out, N)
-        d_e = self.d_e[:E]
-        d_e.zero_()
+        base = self.grad.data_ptr()
+        d_h, d_agg, d_e = self.d_h, self.d_agg, self.d_e
+
+        def grads(mlp, inp, dY, add, idx, hid, dX, acc, dH, dYb):
+            _ok(Lb.gnn_mlp_grads(C.byref(inp), C.byref(mlp.weights(F)), ptr(dY), ptr(add), ptr(idx), ptr(hid),
+                                 (C.c_void_p * 3)(*[None if d is None else d.data_ptr() for d in dX]), acc,
+                                 ptr(dH), ptr(dYb), ptr(self.work), GRAD_WORK_FLOATS,
+                                 C.c_void_p(base + 4 * mlp.o_W1), s), "mlp gradients")
+
+        none3 = (None, None, None)
+        grads(self.dec, io(N, (self.h[self.L], None)), d_out, None, None, self.hid_dec, (d_h, None, None), 0,
+              self.dH_n, self.dY_n)
         for l in reversed(range(self.L)):
             h, e = self.h[l], self.e[l]
-            # node MLP: h_{l+1} = h_l + MLP_n([h_l, agg_l])
-            inp = io(N, (h[:N], None), (self.agg[l], None))
-            self._wgrad_w2_only(self.node[l], self.hid_n[l], d_h, N)
-            # accumulate bit 0 only: the residual source adds into d_h, d_agg is overwritten
-            bwd(self.node[l], inp, d_h, self.hid_n[l], self.dH_n[:N], [d_h, self.d_agg[:N], None], 1, N)
-            self._wgrad_w1_only(self.node[l], inp, self.dH_n[:N])
+            # node MLP: h_{l+1} = h_l + MLP_n([h_l, agg_l]); the residual
+            # source adds into d_h (accumulate bit 0), d_agg is overwritten
+            grads(self.node[l], io(N, (h, None), (self.agg[l], None)), d_h, None, None, self.hid_n[l],
+                  (d_h, d_agg, None), 1, self.dH_n, self.dY_n)
             if E > 0:
-                # aggregation: d_e(l+1) += d_agg[recv]
-                _ok(Lb.gnn_broadcast_add(ptr(self.d_agg), ptr(g.recv), E, ptr(d_e), s), "broadcast")
-                # edge MLP: e_{l+1} = e_l + MLP_e([e_l, h_l[recv], h_l[send]])
-                inp = io(E, (e[:E], None), (h, g.recv), (h, g.send))
-                self._wgrad_w2_only(self.edge[l], self.hid_e[l], d_e, E)
-                bwd(self.edge[l], inp, d_e, self.hid_e[l], self.dH_e[:E],
-                    [d_e, self.d_hi[:E], self.d_hj[:E]], 1, E)
-                self._wgrad_w1_only(self.edge[l], inp, self.dH_e[:E])
-                _ok(Lb.gnn_edge_grad_to_nodes(ptr(self.d_hi), ptr(self.d_hj), ptr(g.row), ptr(g.rev), N,
-                                              ptr(d_h), s), "edge grads to nodes")
+                # edge MLP: e_{l+1} = e_l + MLP_e([e_l, h_l[recv], h_l[send]]),
+                # aggregated into agg_l: d_e(l+1) += d_agg[recv] on the way in
+                # (nothing but that for the last layer)
+                grads(self.edge[l], io(E, (e, None), (h, g.recv), (h, g.send)), d_e if l + 1 < self.L else None,
+                      d_agg, g.recv, self.hid_e[l], (d_e, None, None), 1, self.dH_e, self.dY_e)
+                _ok(Lb.gnn_edge_hidden_grad_to_nodes(N, ptr(self.dH_e), ptr(g.row), ptr(g.rev),
+                                                     C.byref(self.edge[l].weights(F)), ptr(d_h), s),
+                    "edge grads to nodes")
         # encoders (their inputs are data: no input gradient)
         if E > 0:
-            inp = io(E, (xe, None))
-            self._wgrad_w2_only(self.enc_e, self.hid_enc_e, d_e, E)
-            bwd(self.enc_e, inp, d_e, self.hid_enc_e, self.dH_e[:E], [None, None, None], 0, E)
-            self._wgrad_w1_only(self.enc_e, inp, self.dH_e[:E])
+            grads(self.enc_e, io(E, (xe, None)), d_e, None, None, self.hid_enc_e, none3, 0, self.dH_e, self.dY_e)
         else:
             self._zero_grad(self.enc_e)
             for l in range(self.L):
                 self._zero_grad(self.edge[l])
-        inp = io(N, (xn, None))
-        self._wgrad_w2_only(self.enc_n, self.hid_enc_n, d_h, N)
-        bwd(self.enc_n, inp, d_h, self.hid_enc_n, self.dH_n[:N], [None, None, None], 0, N)
-        self._wgrad_w1_only(self.enc_n, inp, self.dH_n[:N])
+        grads(self.enc_n, io(N, (xn, None)), d_h, None, None, self.hid_enc_n, none3, 0, self.dH_n, self.dY_n)
 
     def _zero_grad(self, mlp):
         self.grad[mlp.o_W1:mlp.end].zero_()
-
-    def _wgrad_w2_only(self, mlp, hid, dY32, M):
-        base = self.grad.data_ptr()
-        _ok(glib().gnn_weight_grad(C.byref(io(M, (hid[:M], None))), None, ptr(dY32), mlp.nout, mlp.NP,
-                                   ptr(self.part), ptr(self.bpart), self.nchunks,
-                                   C.c_void_p(base + 4 * mlp.o_W2), C.c_void_p(base + 4 * mlp.o_b2), 0,
-                                   stream()), "wgrad W2")
-
-    def _wgrad_w1_only(self, mlp, inp, dH):
-        base = self.grad.data_ptr()
-        _ok(glib().gnn_weight_grad(C.byref(inp), ptr(dH), None, LAT, LAT, ptr(self.part), ptr(self.bpart),
-                                   self.nchunks, C.c_void_p(base + 4 * mlp.o_W1),
-                                   C.c_void_p(base + 4 * mlp.o_b1), 0, stream()), "wgrad W1")
 
 
 def mse(pred, target):

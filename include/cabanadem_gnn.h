@@ -76,6 +76,29 @@ int gnn_mlp_backward(const gnn_mlp_io* io, const gnn_mlp_weights* w, const float
 int gnn_weight_grad(const gnn_mlp_io* io, const void* G_bf16, const float* G_f32, int ncols,
                     int ncols_pad, float* part, float* bpart, int nchunks, float* dW, float* db,
                     int accumulate, void* stream);
+/* The whole backward of one MLP of the network, parameter gradients included
+ * (up to the FP32 order of those sums the same as gnn_broadcast_add,
+ * gnn_mlp_backward and two gnn_weight_grad):
+ *   dY' = dY + add[add_idx]  (add: float [.][128], NULL: none; dY NULL: zero),
+ *   dH = (dY' W2^T) masked by hidden > 0, bf16 [M][128];  dYb = dY' as bf16
+ *   [M][nout_pad] (both outputs: work arrays of the caller's),
+ *   dX[q] (float [M][128], NULL to skip, two at most) = dH W1^T restricted to
+ *   source q, stored, or added when bit q of accumulate is set; a source whose
+ *   dX is dY (or dY NULL) gets dY' + dH W1^T, as a residual does,
+ *   grad = W1 [K][128] | b1 [128] | W2 [128][nout_pad] | b2 [nout_pad].
+ * Sources: each 128 wide (gathered or not), or one of 32 without dX; 128
+ * outputs, or up to 16 (nout_pad 16, no add).  Arrays 16-byte aligned.
+ * work: GNN_GRAD_WORK_FLOATS floats cover every shape on a GPU of up to 256
+ * compute units.  Deterministic. */
+#define GNN_GRAD_WORK_FLOATS (5L * 1024L * 1024L)
+int gnn_mlp_grads(const gnn_mlp_io* io, const gnn_mlp_weights* w, const float* dY, const float* add,
+                  const int* add_idx, const void* hidden, float* const dX[3], int accumulate, void* dH,
+                  void* dYb, float* work, long work_floats, float* grad, void* stream);
+/* The edge MLP's gradients at the nodes it gathered: dh[i] (float [N][128])
+ * += sum over the edges e of i, in order, of dH[e] W1b^T + dH[rev[e]] W1c^T,
+ * dH (bf16 [E][128]) from gnn_mlp_grads of the edge MLP w (K = 384). */
+int gnn_edge_hidden_grad_to_nodes(int N, const void* dH, const int* row, const int* rev,
+                                  const gnn_mlp_weights* w, float* dh, void* stream);
 /* agg[i] (bf16 [N][128]) = sum of x[e] (bf16 [E][128]) over the edges
  * e in [row[i], row[i+1]), summed in FP32. */
 int gnn_segment_sum(const void* x, const int* row, int N, void* agg, void* stream);
