@@ -20,7 +20,7 @@ ORACLE_DIR = ROOT / "oracle"
 # the force kernels are instantiated per tile size in three translation units
 # (dem_force*.hip), compiled in parallel with the others
 HIP_SOURCES = ["dem_api.hip", "dem_build.hip", "dem_force.hip", "dem_force_b64.hip",
-               "dem_force_b256.hip", "dem_gen.cpp"]
+               "dem_force_b256.hip", "dem_force_group.hip", "dem_gen.cpp"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

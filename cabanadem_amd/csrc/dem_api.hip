@@ -229,6 +229,7 @@ struct dem_ctx {
     a.tiles = nsys > 1 ? d_tiles : nullptr;
     a.ntiles = ntiles;
     a.block = kForceBlocks[bonds_on ? 1 : bidx];
+    a.sysid = d_sysid;
     a.xr_in = xr[cP]; a.xr_out = xr[cP ^ 1];
     a.uw_in = uw[cP]; a.uw_out = uw[cP ^ 1];
     a.mat = mat[cS]; a.mI = mI[cS]; a.ft = ft[cS];

@@ -78,11 +78,11 @@ __device__ inline void store6(double* p, const double* v) {
 // Particle-particle contact of i with j (overlap > 0 already established).
 // h is the tangential history of (i, j), updated in place.  F (and, in
 // corrected mode, T) accumulate.  Line numbers: src/CabanaDEM_Force.hpp.
-template <bool REF>
+template <bool REF, class Params>
 __device__ inline void pp_contact(const double4& xi, const double* ui, const double4& mi,
                                   const double4& xj, const double* uj, const double4& mj,
                                   double* h, double* F, double* T, const StepArgs& a,
-                                  const SysParams& P) {
+                                  const Params& P) {
   const double p0 = xi.x - xj.x, p1 = xi.y - xj.y, p2 = xi.z - xj.z; // :94-96
   const double r2 = p0 * p0 + p1 * p1 + p2 * p2;                      // :99
   const double rij = sqrt(r2);                                        // :101
@@ -171,10 +171,10 @@ __device__ inline void pp_contact(const double4& xi, const double* ui, const dou
 // Particle-wall contact (overlap > 0 already established).  sw is the
 // wall tangential history, updated in place.  src/CabanaDEM_Force.hpp.
 // wx: the wall point at this force pass (moved in corrected mode).
-template <bool REF>
+template <bool REF, class Params>
 __device__ inline void pw_contact(const double4& xi, const double* ui, const double4& mi,
                                   const WallConst& W, const double* wx, double overlap, double* sw,
-                                  double* F, double* T, const StepArgs& a, const SysParams& P) {
+                                  double* F, double* T, const StepArgs& a, const Params& P) {
   const double nx = W.n[0], ny = W.n[1], nz = W.n[2];               // :509-511
   const double a_i = xi.w - overlap / 2.;                           // :517
   double v0, v1, v2;

@@ -145,6 +145,7 @@ struct StepArgs {
   const int4* tiles;
   int ntiles;
   int block;
+  const int* sysid;      // [n] system of each slot (ensembles; null: one system)
 
   const double4* xr_in;
   double4* xr_out;
@@ -287,6 +288,15 @@ enum ForceKind {
 // persistent grid that strides over the tiles.
 hipError_t launch_force(ForceKind kind, const StepArgs& a, bool sample, int grid_blocks,
                         hipStream_t s);
+// The same whole force passes (FK_PP_PW_FORCES, FK_STEP_FUSED, FK_STEP_LAST)
+// with eight lanes per particle, for systems without bonds and groups
+// (dem_force_group.hip); bitwise the same results.
+hipError_t launch_force_group(bool ref, ForceKind kind, const StepArgs& a, hipStream_t s);
+// Particles up to which the eight-lane pass is the faster one.
+#ifndef DEM_GROUP_MAX
+#define DEM_GROUP_MAX 20000
+#endif
+constexpr int kGroupMax = DEM_GROUP_MAX;
 hipError_t launch_zero_forces(const StepArgs& a, hipStream_t s);
 hipError_t launch_update_tangential(const StepArgs& a, hipStream_t s);
 hipError_t launch_set_kinematics(int n, const int* id, const double* x, const double* u, int clear,

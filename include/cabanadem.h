@@ -326,8 +326,9 @@ int dem_set_system_params(dem_ctx* ctx, int system, double cor_pp, double cor_pw
 /* out[s][5] = KE_trans, KE_rot, px, py, pz of each system, current state. */
 int dem_system_diagnostics(dem_ctx* ctx, double* out);
 /* Force-kernel launch shape: grid_blocks = 0 launches one workgroup per
- * tile of 128 particles; > 0 launches a persistent grid of that many
- * workgroups that stride over the tiles.  Results do not depend on it. */
+ * tile of 128 particles (up to 20,000 particles in the default force pass: one
+ * per 16, eight lanes to a particle); > 0 launches a persistent grid of that
+ * many workgroups that stride over the tiles.  Results do not depend on it. */
 int dem_set_launch(dem_ctx* ctx, int grid_blocks);
 /* Force-pass shape (systems without bonds).  Results are bitwise the same
  * in every shape; which is fastest depends on the contact density.
