@@ -112,6 +112,34 @@ __global__ __launch_bounds__(kBlock) void k_kick(StepArgs a, double4* xr, double
   }
 }
 
+__global__ __launch_bounds__(1024) void k_sample_lists(int n, const int* cmeta, const int* nbond, DevFlags* flags) {
+  __shared__ int part[2][16];
+  int c = 0, b = 0;
+#pragma unroll
+  for (int k = 0; k < kListSamples / 1024; ++k) {
+    const long i = (long)(k * 1024 + threadIdx.x) * n / kListSamples;
+    c += meta_count(cmeta[i]);
+    if (nbond) b += nbond[i];
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    c += __shfl_xor(c, off);
+    b += __shfl_xor(b, off);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    part[0][threadIdx.x >> 6] = c;
+    part[1][threadIdx.x >> 6] = b;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < 16; ++k) {
+      c += part[0][k];
+      b += part[1][k];
+    }
+    flags->sampled_contacts = c;
+    flags->sampled_bonds = b;
+  }
+}
+
 template <int B>
 __global__ __launch_bounds__(B) void k_diag_current(StepArgs a, const double* uw) {
   const int tile = blockIdx.x;
@@ -238,6 +266,11 @@ hipError_t launch_update_tangential(const StepArgs& a, hipStream_t s) {
 hipError_t launch_kick(const StepArgs& a, double4* xr, double* uw, const double* ft,
                        int do_kick, int do_drift, hipStream_t s) {
   hipLaunchKernelGGL(k_kick, dim3(nblk(a.n)), dim3(kBlock), 0, s, a, xr, uw, ft, do_kick, do_drift);
+  return hipGetLastError();
+}
+
+hipError_t launch_sample_lists(int n, const int* cmeta, const int* nbond, DevFlags* flags, hipStream_t s) {
+  hipLaunchKernelGGL(k_sample_lists, dim3(1), dim3(1024), 0, s, n, cmeta, nbond, flags);
   return hipGetLastError();
 }
 

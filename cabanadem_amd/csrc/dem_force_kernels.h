@@ -38,12 +38,13 @@ namespace {
 #ifndef DEM_FORCE_MIN_WAVES
 #define DEM_FORCE_MIN_WAVES 1
 #endif
-// The corrected arithmetic's force kernels would take about 150 VGPRs (3
-// waves per SIMD); held to 128 (4 waves, a few spilled values) they are 4 %
-// faster on contact-dense beds.  The bonded and sampling variants spill far
-// more at 128 and stay unbounded.
-#ifndef DEM_FORCE_MIN_WAVES_CORRECTED
-#define DEM_FORCE_MIN_WAVES_CORRECTED 4
+// Whole passes without bonds or sampling are held to 128 VGPRs (4 waves per
+// SIMD, a few spilled values).  Left alone the compiler takes 150 to 160 (3
+// waves): 4 % slower on the contact-dense bed with the corrected arithmetic,
+// 6 % on the 4M bed with the reference's.  The bonded and sampling variants
+// spill far more at 128 and stay unbounded.
+#ifndef DEM_FORCE_MIN_WAVES_PLAIN
+#define DEM_FORCE_MIN_WAVES_PLAIN 4
 #endif
 constexpr int kPhase1Batch = DEM_PHASE1_BATCH; // neighbour gathers issued together
 #ifndef DEM_DETECT_BATCH
@@ -456,15 +457,55 @@ __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Bytes of dynamic LDS per workgroup of B threads: the contact ids found in
-// phase 1 (int [max_c][B]), for the wave/tile pass also the old slot of each
-// (byte [max_c][B], padded to 8), the contact shares (double [B][6]) and the
-// lanes' first contact numbers (int [B]).
+// A wave's own region of dynamic LDS, in ints: the contact ids found in phase
+// 1 (int [max_c][64]), and at the end the staging of its 64 particles' new
+// state (80 bytes each).
+__host__ __device__ inline int wave_region(int max_c) {
+  const int ids = (max_c > 0 ? max_c : 1) * 64, stage = 64 * 80 / 4;
+  return ids > stage ? ids : stage;
+}
+
+// Bytes of dynamic LDS per workgroup of B threads: the waves' regions, for
+// the wave/tile pass also the old slot of each contact (byte [max_c][B],
+// padded to 8), the contact shares (double [B][6]) and the lanes' first
+// contact numbers (int [B]).
 __host__ __device__ inline size_t force_lds_bytes(int max_c, bool wave, int B) {
   const size_t mc = (size_t)(max_c > 0 ? max_c : 1);
-  size_t b = mc * B * sizeof(int);
+  size_t b = (size_t)(B / 64) * wave_region(max_c) * sizeof(int);
   if (wave) b += (mc * B + 7) / 8 * 8 + (size_t)B * 6 * sizeof(double) + (size_t)B * sizeof(int);
   return b;
+}
+
+// Loads and stores of data that no other wave of the launch reads, past the
+// caches where NT is set.
+template <bool NT, class T>
+__device__ __forceinline__ T stream_load(const T* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool NT, class T>
+__device__ __forceinline__ void stream_store(T* p, T v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+template <bool NT>
+__device__ __forceinline__ double2 stream_load2(const double2* p) {
+  if constexpr (NT) return make_double2(__builtin_nontemporal_load(&p->x), __builtin_nontemporal_load(&p->y));
+  else return *p;
+}
+template <bool NT>
+__device__ __forceinline__ void stream_store2(double2* p, double2 v) {
+  if constexpr (NT) {
+    __builtin_nontemporal_store(v.x, &p->x);
+    __builtin_nontemporal_store(v.y, &p->y);
+  } else {
+    *p = v;
+  }
+}
+
+// The contact id of thread t's m-th contact.
+__device__ __forceinline__ int& contact_id(int* s_cj, int max_c, int m, int t) {
+  return s_cj[(t >> 6) * wave_region(max_c) + m * 64 + (t & 63)];
 }
 
 // Particle-particle contact arithmetic spread over the lanes of a wave.
@@ -481,7 +522,7 @@ __host__ __device__ inline size_t force_lds_bytes(int max_c, bool wave, int B) {
 // contacts.  Every lane of the wave must call this (shuffles).
 template <bool REF, bool PRE, int B>
 __device__ __forceinline__ void wave_contacts(const StepArgs& a, const SysParams& P, const int first,
-                                              const int nc, const int* s_cj, const unsigned char* s_op,
+                                              const int nc, int* s_cj, const unsigned char* s_op,
                                               double* s_con, double* F, double* T) {
   const int tid = threadIdx.x, lane = tid & 63, wbase = tid - lane;
   const long ld = a.ld;
@@ -507,7 +548,7 @@ __device__ __forceinline__ void wave_contacts(const StepArgs& a, const SysParams
       const int m = k - eL;
       const int o = wbase + L; // the owner's thread in the workgroup
       const int io = first + o;
-      const int j = PRE ? a.cj_out[m * ld + io] : s_cj[m * B + o];
+      const int j = PRE ? a.cj_out[m * ld + io] : contact_id(s_cj, a.max_c, m, o);
       const int p1 = s_op[m * B + o];
       double h[3] = {0., 0., 0.};
       if (p1 > 0) { // continued contact: src/CabanaDEM_Force.hpp:166-178
@@ -554,7 +595,7 @@ __device__ __forceinline__ void wave_contacts(const StepArgs& a, const SysParams
 // of the workgroup must call this (barriers).
 template <bool REF, bool PRE, int B>
 __device__ __forceinline__ void tile_contacts(const StepArgs& a, const SysParams& P, const int first,
-                                              const int nc, const int* s_cj, const unsigned char* s_op,
+                                              const int nc, int* s_cj, const unsigned char* s_op,
                                               double* s_con, int* s_ex, double* F, double* T) {
   if constexpr (B == 64) {
     wave_contacts<REF, PRE, B>(a, P, first, nc, s_cj, s_op, s_con, F, T);
@@ -591,7 +632,7 @@ __device__ __forceinline__ void tile_contacts(const StepArgs& a, const SysParams
           if (s_ex[L + st] <= k) L += st;
         const int m = k - s_ex[L];
         const int io = first + L;
-        const int j = PRE ? a.cj_out[m * ld + io] : s_cj[m * B + L];
+        const int j = PRE ? a.cj_out[m * ld + io] : contact_id(s_cj, a.max_c, m, L);
         const int p1 = s_op[m * B + L];
         double h[3] = {0., 0., 0.};
         if (p1 > 0) { // continued contact: src/CabanaDEM_Force.hpp:166-178
@@ -635,7 +676,7 @@ __device__ __forceinline__ void tile_contacts(const StepArgs& a, const SysParams
 // One tile: B consecutive slots of one system.  ENS: an ensemble (tile
 // table and per-system parameters from the device); otherwise one system
 // whose parameters travel in the kernel arguments.  Each lane walks its own
-// contact list, or (a.wave, systems without bonds) the tile runs the contact
+// contact list, or (WAVE, systems without bonds) the tile runs the contact
 // arithmetic of all its lanes spread over the lanes (tile_contacts).
 // PASS (systems without bonds, whole force passes, no sampling):
 //   0  everything in one pass;
@@ -649,13 +690,16 @@ __device__ __forceinline__ void tile_contacts(const StepArgs& a, const SysParams
 //      (ids in cj_out); a tile with an empty list returns at once.
 // Every particle's arithmetic is that of PASS 0, so the results are bitwise
 // the same.
+// NT: the launch's own streams (rows, counts, m and I, the contact lists and
+// histories of the lane walk, the new state) go past the caches, which keep
+// what neighbours gather.
 template <bool REF, bool PP, bool PW, int KICK, bool ACCUM, bool DIAG, bool BOND, bool ENS, bool PRE, int B,
-          int PASS = 0>
+          int PASS = 0, bool NT = false, bool WAVE = false>
 __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, int* s_cj) {
   constexpr bool DEFER = PASS == 1, LIST = PASS == 2;
   static_assert(PASS == 0 || (PP && PW && !ACCUM && !DIAG && !BOND), "deferral: whole passes only");
   static_assert(!LIST || PRE, "the work-list pass reads its contact ids from cj_out");
-  constexpr bool WAVE = PP && !BOND && PASS == 0;
+  static_assert(!WAVE || (PP && !BOND && PASS == 0), "the wave pass: contacts of systems without bonds");
   const int tid = threadIdx.x;
   int sys = 0, first = tile * B, end = a.n;
   int i;
@@ -676,10 +720,21 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
   }
   const SysParams& P = ENS ? a.sys[sys] : a.sys0;
   const long ld = a.ld;
-  unsigned char* s_op = reinterpret_cast<unsigned char*>(s_cj + (long)(a.max_c > 0 ? a.max_c : 1) * B);
+  unsigned char* s_op = reinterpret_cast<unsigned char*>(s_cj + (B / 64) * wave_region(a.max_c));
   double* s_con = reinterpret_cast<double*>(
       reinterpret_cast<char*>(s_cj) + force_lds_bytes(a.max_c, false, B) +
       ((size_t)(a.max_c > 0 ? a.max_c : 1) * B + 7) / 8 * 8);
+  // The new state leaves through the wave's LDS region, so that every store
+  // instruction covers 1 KB of consecutive memory.  Stored lane by lane (two
+  // 16-byte pieces 32 bytes apart for xr, three 48 apart for uw) each
+  // instruction sent 16 bytes to every 64-byte sector it touched: 208 write
+  // requests a wave instead of 80, of 388 requests in all, and the L2 request
+  // rate is what the pass runs against (4M spheres, settled: 260 -> 243 us;
+  // the same for the loads, whose repeats the L1 absorbs, bought nothing).
+  // The bonded kernels would spill for it.
+  constexpr bool STAGE = PASS == 0 && KICK != 0 && !BOND;
+  const int lane = tid & 63;
+  double2* const stage = reinterpret_cast<double2*>(s_cj + (tid >> 6) * wave_region(a.max_c));
   double dg[8] = {0., 0., 0., 0., 0., 0., 0., 0.};
   double cd2 = 0., cv2 = 0.; // displacement check terms (a.disp)
   double4 xi = make_double4(0., 0., 0., 0.);
@@ -691,14 +746,14 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
   double F[3] = {0., 0., 0.}, T[3] = {0., 0., 0.};
   int meta = 0, nnb = 0, nc = 0, nwc = 0;
   // in a bonded run, contacts only between unbonded pairs (or none at all)
-  const bool pp_on = !a.nbond || a.unbonded_contacts;
+  const bool pp_on = (!BOND && !ACCUM) || !a.nbond || a.unbonded_contacts;
   if (act) {
     xi = a.xr_in[i];
     // loaded here, in flight over phase 1 (the deferral pass too, unless
     // DEM_DEFER_EARLY_LOADS is 0: fewer registers, one more round trip)
     if (!DEFER || DEM_DEFER_EARLY_LOADS) {
       load6(a.uw_in + 6l * i, ui);
-      mI = a.mI[i];
+      mI = stream_load2<NT>(a.mI + i);
     }
     if (DEFER) {
     } else if (ACCUM) {
@@ -719,22 +774,22 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
         if (j < 0) continue;
         double h[9];
 #pragma unroll
-        for (int c = 0; c < 9; ++c) h[c] = a.bh[(9 * b + c) * ld + i];
+        for (int c = 0; c < 9; ++c) h[c] = stream_load<NT>(a.bh + (9 * b + c) * ld + i);
         const double4 xj = a.xr_in[j];
         double uj[6];
         load6(a.uw_in + 6l * j, uj);
-        if (bond_force<REF>(xi, ui, EGi, xj, uj, a.bl[(long)b * ld + i], h, F, T, a)) {
+        if (bond_force<REF>(xi, ui, EGi, xj, uj, stream_load<NT>(a.bl + (long)b * ld + i), h, F, T, a)) {
           a.bj[(long)b * ld + i] = -1;
           atomicAdd(&a.flags->bonds_broken, 1);
           continue;
         }
 #pragma unroll
-        for (int c = 0; c < 9; ++c) a.bh[(9 * b + c) * ld + i] = h[c];
+        for (int c = 0; c < 9; ++c) stream_store<NT>(a.bh + (9 * b + c) * ld + i, h[c]);
       }
     }
-    meta = a.cmeta_in[i];
+    meta = stream_load<NT>(a.cmeta_in + i);
     nc = meta_count(meta);
-    const int nbk = a.nbond ? (BOND ? nb : a.nbond[i]) : 0;
+    const int nbk = (BOND || ACCUM) && a.nbond ? (BOND ? nb : a.nbond[i]) : 0;
     if (PP && !pp_on) nc = 0;
     if (PP && pp_on && PRE) {
       // Phase 1 ran in k_detect: the count is in cmeta_out, the ids (ascending)
@@ -749,8 +804,8 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
       // bounds whatever the count, and the count masks them afterwards.
       int jr0[NB];
 #pragma unroll
-      for (int q = 0; q < NB; ++q) jr0[q] = (q < a.max_n) ? a.nbr[q * ld + i] : i;
-      nnb = a.nn[i];
+      for (int q = 0; q < NB; ++q) jr0[q] = (q < a.max_n) ? stream_load<NT>(a.nbr + q * ld + i) : i;
+      nnb = stream_load<NT>(a.nn + i);
       nc = 0;
       // Batches of NB independent row loads, then gathers, then
       // tests: several gathers in flight per lane instead of one chain.
@@ -762,7 +817,7 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
           for (int q = 0; q < NB; ++q) jb[q] = (q < nnb) ? jr0[q] : i;
         } else {
 #pragma unroll
-          for (int q = 0; q < NB; ++q) jb[q] = (k0 + q < nnb) ? a.nbr[(k0 + q) * ld + i] : i;
+          for (int q = 0; q < NB; ++q) jb[q] = (k0 + q < nnb) ? stream_load<NT>(a.nbr + (k0 + q) * ld + i) : i;
         }
 #pragma unroll
         for (int q = 0; q < NB; ++q) xb[q] = a.xr_in[jb[q]];
@@ -779,7 +834,7 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
             if (s - sqrt(r2) > 0. && !(nbk > 0 && bonded_to(a, i, nbk, jb[q]))) {
               if (nc < a.max_c) {
                 if (DEFER) a.cj_out[nc * ld + i] = jb[q];
-                else s_cj[nc * B + tid] = jb[q];
+                else contact_id(s_cj, a.max_c, nc, tid) = jb[q];
               }
               ++nc;
             }
@@ -791,7 +846,7 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
         nc = a.max_c;
       }
     }
-    if (WAVE && pp_on && a.wave) {
+    if (WAVE && pp_on) {
       // merge with last step's tracked list (both ascending in j): the old
       // slot of each contact, or 0 for a new one
       // (src/CabanaDEM_Force.hpp:166-192, 399-433)
@@ -799,7 +854,7 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
       int p = 0;
       int jo = oc > 0 ? a.cj_in[i] : INT_MAX;
       for (int m = 0; m < nc; ++m) {
-        const int j = PRE ? a.cj_out[m * ld + i] : s_cj[m * B + tid];
+        const int j = PRE ? a.cj_out[m * ld + i] : contact_id(s_cj, a.max_c, m, tid);
         while (jo < j) {
           ++p;
           jo = (p < oc) ? a.cj_in[p * ld + i] : INT_MAX;
@@ -808,8 +863,7 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
       }
     }
   }
-  const bool wave = WAVE && pp_on && a.wave; // uniform over the launch
-  if (wave) {
+  if (WAVE && pp_on) {
     // every lane of the tile, active or not: the contacts of the tile
     wave_lds_sync();
     tile_contacts<REF, PRE, B>(a, P, first, act ? nc : 0, s_cj, s_op, s_con,
@@ -819,29 +873,29 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
     // contact arithmetic, merged with last step's tracked list.
     const int oc = meta_count(meta);
     int p = 0;
-    int jo = oc > 0 ? a.cj_in[i] : INT_MAX;
+    int jo = oc > 0 ? stream_load<NT>(a.cj_in + i) : INT_MAX;
     if (nc > 0) { mti = a.mat[i]; have_mti = true; }
     for (int m = 0; m < nc; ++m) {
-      const int j = PRE ? a.cj_out[m * ld + i] : s_cj[m * B + tid];
+      const int j = PRE ? a.cj_out[m * ld + i] : contact_id(s_cj, a.max_c, m, tid);
       while (jo < j) {
         ++p;
-        jo = (p < oc) ? a.cj_in[p * ld + i] : INT_MAX;
+        jo = (p < oc) ? stream_load<NT>(a.cj_in + p * ld + i) : INT_MAX;
       }
       double h[3] = {0., 0., 0.};
       if (jo == j) {
-        h[0] = a.ch_in[(3 * p + 0) * ld + i];
-        h[1] = a.ch_in[(3 * p + 1) * ld + i];
-        h[2] = a.ch_in[(3 * p + 2) * ld + i];
+        h[0] = stream_load<NT>(a.ch_in + (3 * p + 0) * ld + i);
+        h[1] = stream_load<NT>(a.ch_in + (3 * p + 1) * ld + i);
+        h[2] = stream_load<NT>(a.ch_in + (3 * p + 2) * ld + i);
       }
       const double4 xj = a.xr_in[j];
       double uj[6];
       load6(a.uw_in + 6l * j, uj);
       const double4 mj = a.mat[j];
       pp_contact<REF>(xi, ui, mti, xj, uj, mj, h, F, T, a, P);
-      if (!PRE) a.cj_out[m * ld + i] = j;
-      a.ch_out[(3 * m + 0) * ld + i] = h[0];
-      a.ch_out[(3 * m + 1) * ld + i] = h[1];
-      a.ch_out[(3 * m + 2) * ld + i] = h[2];
+      if (!PRE) stream_store<NT>(a.cj_out + m * ld + i, j);
+      stream_store<NT>(a.ch_out + (3 * m + 0) * ld + i, h[0]);
+      stream_store<NT>(a.ch_out + (3 * m + 1) * ld + i, h[1]);
+      stream_store<NT>(a.ch_out + (3 * m + 2) * ld + i, h[2]);
     }
   }
   bool defer = false;
@@ -914,7 +968,7 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
       }
     }
     if (DEFER) wn = 0; // no wall overlaps: any old history is dropped
-    if (PP) a.cmeta_out[i] = make_meta(nc, wn);
+    if (PP) stream_store<NT>(a.cmeta_out + i, make_meta(nc, wn));
     else if (PW) a.cmeta_in[i] = make_meta(nc, wn); // walls only: in place
     if (!ACCUM) apply_force_bc(a, i, F);
     if (KICK == 0) {
@@ -929,6 +983,7 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
       // 1/m and 1/I per use, src/CabanaDEM_Integrator.hpp:42,48
       const double minv = 1. / mI.x, Iinv = 1. / mI.y;
       double s[6];
+      double4 xo;
       // stage3: src/CabanaDEM_Integrator.hpp:89-98
       s[0] = ui[0] + a.hdt * F[0] * minv;
       s[1] = ui[1] + a.hdt * F[1] * minv;
@@ -947,25 +1002,43 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
         for (int d = 0; d < 3; ++d) s[d] = s[d] + a.hdt * F[d] * minv;
         for (int d = 0; d < 3; ++d) s[3 + d] = s[3 + d] + a.hdt * T[d] * Iinv;
         apply_vgroup(a, i, s);
-        double4 xo;
         xo.x = xi.x + a.dt * s[0];
         xo.y = xi.y + a.dt * s[1];
         xo.z = xi.z + a.dt * s[2];
         xo.w = xi.w;
-        a.xr_out[i] = xo;
-        store6(a.uw_out + 6l * i, s);
         if (a.disp) disp_terms(a, i, xo, s, cd2, cv2);
       } else {
-        a.xr_out[i] = xi;
-        store6(a.uw_out + 6l * i, s);
+        xo = xi;
         double ft[6] = {F[0], F[1], F[2], T[0], T[1], T[2]};
         store6(a.ft + 6l * i, ft);
         if (a.disp) disp_terms(a, i, xi, s, cd2, cv2);
+      }
+      if (STAGE) {
+        stage[2 * lane] = make_double2(xo.x, xo.y);
+        stage[2 * lane + 1] = make_double2(xo.z, xo.w);
+        store6(reinterpret_cast<double*>(stage + 128 + 3 * lane), s);
+      } else {
+        a.xr_out[i] = xo;
+        store6(a.uw_out + 6l * i, s);
       }
     }
     dg[5] = (double)nnb;
     dg[6] = (double)nc;
     dg[7] = (double)nwc;
+  }
+  if (STAGE) {
+    const int w0 = first + tid - lane;
+    const int cnt = min(64, end - w0); // the wave's particles (none: negative)
+    wave_lds_sync();
+    double2* gx = reinterpret_cast<double2*>(a.xr_out + w0);
+    double2* gu = reinterpret_cast<double2*>(a.uw_out + 6l * w0);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (k * 64 + lane < 2 * cnt) stream_store2<NT>(gx + k * 64 + lane, stage[k * 64 + lane]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (k * 64 + lane < 3 * cnt) stream_store2<NT>(gu + k * 64 + lane, stage[128 + k * 64 + lane]);
+    wave_lds_sync(); // a persistent grid's next tile writes its contacts there
   }
   if (DIAG) block_reduce8<B>(dg, a.diag_part, tile);
   if (KICK != 0 && a.disp) disp_block_max<B>(cd2, cv2, a.disp);
@@ -974,19 +1047,21 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
 // The fused force / step kernel.  A grid of one workgroup per tile, or a
 // persistent grid that strides over the tiles; either way tile v is mapped
 // XCD-aware (contiguous tiles per XCD when the grid is a multiple of 8).
-template <bool REF, bool PP, bool PW, int KICK, bool ACCUM, bool DIAG, bool BOND, bool ENS, bool PRE, int B>
+template <bool REF, bool PP, bool PW, int KICK, bool ACCUM, bool DIAG, bool BOND, bool ENS, bool PRE, int B,
+          bool NT, bool WAVE>
 __global__ __launch_bounds__(B, PRE ? DEM_PRE_MIN_WAVES
-                                 : (!REF && !BOND && !DIAG) ? DEM_FORCE_MIN_WAVES_CORRECTED : DEM_FORCE_MIN_WAVES)
+                                 : (!BOND && !DIAG) ? DEM_FORCE_MIN_WAVES_PLAIN : DEM_FORCE_MIN_WAVES)
 void k_force(StepArgs a) {
-  extern __shared__ int s_cj[]; // [max_c][B] contacts found in phase 1
+  extern __shared__ __attribute__((aligned(16))) int s_cj[]; // the waves' regions, then the wave pass's columns
   if ((int)gridDim.x >= a.ntiles) {
     // one workgroup per tile: no loop, so the compiler keeps the kernel
     // arguments where they are used instead of live across a loop
-    force_tile<REF, PP, PW, KICK, ACCUM, DIAG, BOND, ENS, PRE, B>(a, xcd_block(blockIdx.x, a.ntiles), s_cj);
+    force_tile<REF, PP, PW, KICK, ACCUM, DIAG, BOND, ENS, PRE, B, 0, NT, WAVE>(a, xcd_block(blockIdx.x, a.ntiles),
+                                                                                s_cj);
     return;
   }
   for (int v = blockIdx.x; v < a.ntiles; v += gridDim.x) {
-    force_tile<REF, PP, PW, KICK, ACCUM, DIAG, BOND, ENS, PRE, B>(a, xcd_block(v, a.ntiles), s_cj);
+    force_tile<REF, PP, PW, KICK, ACCUM, DIAG, BOND, ENS, PRE, B, 0, NT, WAVE>(a, xcd_block(v, a.ntiles), s_cj);
     if (DIAG) __syncthreads(); // the reduction's LDS is reused by the next tile
   }
 }
@@ -1081,26 +1156,23 @@ __global__ __launch_bounds__(B, 8) void k_detect(StepArgs a) {
 
 inline unsigned nblk(long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
-// The split force pass: k_detect, then the force kernel over its lists.
-// Whole force passes of systems without bonds only; the result is bitwise
-// that of the fused kernel.
+// The split force pass where it samples: k_detect, then the force kernel over
+// its lists.  Whole force passes of systems without bonds only; the result is
+// bitwise that of the fused kernel.
 template <bool REF, bool ENS, int B>
-hipError_t launch_split(ForceKind kind, const StepArgs& a, bool sample, const dim3& g, hipStream_t s) {
+hipError_t launch_split(ForceKind kind, const StepArgs& a, const dim3& g, hipStream_t s) {
   const dim3 b(B);
   const size_t lds = force_lds_bytes(a.max_c, true, B);
   hipLaunchKernelGGL((k_detect<ENS, B>), g, b, 0, s, a);
   switch (kind) {
     case FK_PP_PW_FORCES:
-      if (sample) hipLaunchKernelGGL((k_force<REF, true, true, 0, false, true, false, ENS, true, B>), g, b, lds, s, a);
-      else hipLaunchKernelGGL((k_force<REF, true, true, 0, false, false, false, ENS, true, B>), g, b, lds, s, a);
+      hipLaunchKernelGGL((k_force<REF, true, true, 0, false, true, false, ENS, true, B, false, true>), g, b, lds, s, a);
       break;
     case FK_STEP_FUSED:
-      if (sample) hipLaunchKernelGGL((k_force<REF, true, true, 2, false, true, false, ENS, true, B>), g, b, lds, s, a);
-      else hipLaunchKernelGGL((k_force<REF, true, true, 2, false, false, false, ENS, true, B>), g, b, lds, s, a);
+      hipLaunchKernelGGL((k_force<REF, true, true, 2, false, true, false, ENS, true, B, false, true>), g, b, lds, s, a);
       break;
     case FK_STEP_LAST:
-      if (sample) hipLaunchKernelGGL((k_force<REF, true, true, 1, false, true, false, ENS, true, B>), g, b, lds, s, a);
-      else hipLaunchKernelGGL((k_force<REF, true, true, 1, false, false, false, ENS, true, B>), g, b, lds, s, a);
+      hipLaunchKernelGGL((k_force<REF, true, true, 1, false, true, false, ENS, true, B, false, true>), g, b, lds, s, a);
       break;
     default:
       return hipErrorInvalidValue;
@@ -1131,47 +1203,57 @@ hipError_t launch_deferred(ForceKind kind, const StepArgs& a, const dim3& g, hip
   return hipGetLastError();
 }
 
-// B: the workgroup size and tile of the launch (kBlock for bonded systems).
-template <bool REF, bool BOND, bool ENS, int B>
-hipError_t launch_force_mode(ForceKind kind, const StepArgs& a, bool sample, int grid_blocks,
-                             hipStream_t s) {
-  // systems without bonds run the wave pass, which needs its LDS columns
-  const size_t lds = force_lds_bytes(a.max_c, !BOND, B);
-  const int nb = (grid_blocks > 0 && grid_blocks < a.ntiles) ? grid_blocks : a.ntiles;
-  const dim3 g(nb), b(B);
-  if constexpr (!BOND) {
-    if (a.split && (kind == FK_PP_PW_FORCES || kind == FK_STEP_FUSED || kind == FK_STEP_LAST)) {
-      if (sample) return launch_split<REF, ENS, B>(kind, a, sample, g, s);
-      return launch_deferred<REF, ENS, B>(kind, a, g, s);
-    }
-  }
+// One fused kernel per force pass.  WAVE: the tile spreads its contacts over
+// its lanes (systems without bonds).
+template <bool REF, bool BOND, bool ENS, int B, bool WAVE>
+hipError_t launch_fused(ForceKind kind, const StepArgs& a, bool sample, const dim3& g, hipStream_t s) {
+  const dim3 b(B);
+  const size_t lds = force_lds_bytes(a.max_c, WAVE, B);
   switch (kind) {
     case FK_PP_PW_FORCES:
-      if (sample) hipLaunchKernelGGL((k_force<REF, true, true, 0, false, true, BOND, ENS, false, B>), g, b, lds, s, a);
-      else hipLaunchKernelGGL((k_force<REF, true, true, 0, false, false, BOND, ENS, false, B>), g, b, lds, s, a);
+      if (sample) hipLaunchKernelGGL((k_force<REF, true, true, 0, false, true, BOND, ENS, false, B, false, WAVE>), g, b, lds, s, a);
+      else hipLaunchKernelGGL((k_force<REF, true, true, 0, false, false, BOND, ENS, false, B, false, WAVE>), g, b, lds, s, a);
       break;
     case FK_PP_ACCUM:
-      hipLaunchKernelGGL((k_force<REF, true, false, 0, true, false, false, ENS, false, B>), g, b, lds, s, a);
+      hipLaunchKernelGGL((k_force<REF, true, false, 0, true, false, false, ENS, false, B, false, WAVE>), g, b, lds, s, a);
       break;
     case FK_PW_ACCUM:
-      hipLaunchKernelGGL((k_force<REF, false, true, 0, true, false, false, ENS, false, B>), g, b, lds, s, a);
+      hipLaunchKernelGGL((k_force<REF, false, true, 0, true, false, false, ENS, false, B, false, false>), g, b, lds, s, a);
       break;
     case FK_BOND_ACCUM:
       if constexpr (BOND && !ENS)
-        hipLaunchKernelGGL((k_force<REF, false, false, 0, true, false, true, false, false, B>), g, b, lds, s, a);
+        hipLaunchKernelGGL((k_force<REF, false, false, 0, true, false, true, false, false, B, false, false>), g, b, lds, s, a);
       else
         return hipErrorInvalidValue;
       break;
     case FK_STEP_FUSED:
-      if (sample) hipLaunchKernelGGL((k_force<REF, true, true, 2, false, true, BOND, ENS, false, B>), g, b, lds, s, a);
-      else hipLaunchKernelGGL((k_force<REF, true, true, 2, false, false, BOND, ENS, false, B>), g, b, lds, s, a);
+      if (sample) hipLaunchKernelGGL((k_force<REF, true, true, 2, false, true, BOND, ENS, false, B, false, WAVE>), g, b, lds, s, a);
+      else if (a.stream)
+        hipLaunchKernelGGL((k_force<REF, true, true, 2, false, false, BOND, ENS, false, B, true, WAVE>), g, b, lds, s, a);
+      else hipLaunchKernelGGL((k_force<REF, true, true, 2, false, false, BOND, ENS, false, B, false, WAVE>), g, b, lds, s, a);
       break;
     case FK_STEP_LAST:
-      if (sample) hipLaunchKernelGGL((k_force<REF, true, true, 1, false, true, BOND, ENS, false, B>), g, b, lds, s, a);
-      else hipLaunchKernelGGL((k_force<REF, true, true, 1, false, false, BOND, ENS, false, B>), g, b, lds, s, a);
+      if (sample) hipLaunchKernelGGL((k_force<REF, true, true, 1, false, true, BOND, ENS, false, B, false, WAVE>), g, b, lds, s, a);
+      else hipLaunchKernelGGL((k_force<REF, true, true, 1, false, false, BOND, ENS, false, B, false, WAVE>), g, b, lds, s, a);
       break;
   }
   return hipGetLastError();
+}
+
+// B: the workgroup size and tile of the launch (kBlock for bonded systems).
+template <bool REF, bool BOND, bool ENS, int B>
+hipError_t launch_force_mode(ForceKind kind, const StepArgs& a, bool sample, int grid_blocks,
+                             hipStream_t s) {
+  const int nb = (grid_blocks > 0 && grid_blocks < a.ntiles) ? grid_blocks : a.ntiles;
+  const dim3 g(nb);
+  if constexpr (!BOND) {
+    if (a.split && (kind == FK_PP_PW_FORCES || kind == FK_STEP_FUSED || kind == FK_STEP_LAST)) {
+      if (sample) return launch_split<REF, ENS, B>(kind, a, g, s);
+      return launch_deferred<REF, ENS, B>(kind, a, g, s);
+    }
+    if (a.wave) return launch_fused<REF, false, ENS, B, true>(kind, a, sample, g, s);
+  }
+  return launch_fused<REF, BOND, ENS, B, false>(kind, a, sample, g, s);
 }
 
 } // namespace

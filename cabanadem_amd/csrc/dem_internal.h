@@ -118,7 +118,12 @@ struct DevFlags {
   int bond_overflow;
   int cell_overflow;  // a cell held more than kMaxCellParticles particles
   int bonds_broken;   // bonds broken since the flags were last cleared
+  int sampled_contacts; // tracked contacts and bond slots of kListSamples
+  int sampled_bonds;    // particles (launch policy only)
 };
+
+// Particles whose list lengths the end of a step call samples.
+constexpr int kListSamples = 4096;
 
 // Upper bound on particles in one cell; beyond it the binning box is far too
 // coarse for the cutoff and the rebuild stops with an error instead of
@@ -193,6 +198,9 @@ struct StepArgs {
   // 1: the contact arithmetic of all lanes of a tile runs spread over the
   // tile's lanes (systems without bonds); 0: each lane walks its own list
   int wave;
+  // 1: one fused step touches more than the caches hold, so its own streams
+  // (what no neighbour gathers) go past them; 0: everything is kept
+  int stream;
   // time of this force pass since the walls' positions were set (moving
   // walls, corrected mode)
   double tw;
@@ -305,6 +313,9 @@ hipError_t launch_get_kinematics(int n, const int* id, const double4* xr, const 
                                  double* u, hipStream_t s);
 hipError_t launch_kick(const StepArgs& a, double4* xr, double* uw, const double* ft,
                        int do_kick, int do_drift, hipStream_t s);
+// flags->sampled_contacts, sampled_bonds = those of kListSamples particles
+// spread over the n (nbond null: no bonds).
+hipError_t launch_sample_lists(int n, const int* cmeta, const int* nbond, DevFlags* flags, hipStream_t s);
 // Per-tile partial sums of the current state (one partial row per tile).
 hipError_t launch_diag_current(const StepArgs& a, const double* uw, hipStream_t s);
 // The force kernels for one tile size each (a.block), in translation units
