@@ -148,6 +148,7 @@ struct dem_ctx {
   int* rank = nullptr;
   int* key_sorted = nullptr;
   int* cell_count = nullptr;
+  int* cell_scan = nullptr;
   int* cell_start = nullptr;
   int* perm = nullptr;
   int* inv = nullptr;
@@ -194,7 +195,7 @@ struct dem_ctx {
       hipFree(vgroup[b]); hipFree(fext[b]);
     }
     hipFree(nn); hipFree(nbr); hipFree(xb); hipFree(key); hipFree(rank); hipFree(key_sorted);
-    hipFree(cell_count); hipFree(cell_start); hipFree(perm); hipFree(inv); hipFree(scan_tmp);
+    hipFree(cell_count); hipFree(cell_scan); hipFree(cell_start); hipFree(perm); hipFree(inv); hipFree(scan_tmp);
     hipFree(flags); hipFree(diag_part); hipFree(diag_rows); hipFree(d_disp);
     hipFree(d_work); hipFree(d_work_tile);
     if (h_disp) hipHostFree(h_disp);
@@ -288,6 +289,7 @@ struct dem_ctx {
     BuildArgs b{};
     b.keep_xb = cfg.skin > 0. ? 1 : 0;
     b.permute_ft = permute_ft ? 1 : 0;
+    b.stream = step_bytes(contacts_est, bonds_est) > cache_bytes() ? 1 : 0;
     b.n = n; b.ld = ld; b.max_n = max_n; b.max_c = max_c;
     b.grid = grids[0]; b.ncell = ncell; b.rc2 = rc2;
     if (nsys > 1) { b.sysid = d_sysid; b.grids = d_grids; b.kbase = d_kbase; }
@@ -305,7 +307,7 @@ struct dem_ctx {
     b.cj_in = cj[cC]; b.cj_out = cj[cC ^ 1];
     b.ch_in = ch[cC]; b.ch_out = ch[cC ^ 1];
     b.xb = xb; b.key = key; b.rank = rank; b.key_sorted = key_sorted;
-    b.cell_count = cell_count; b.cell_start = cell_start;
+    b.cell_count = cell_count; b.cell_scan = cell_scan; b.cell_start = cell_start;
     b.perm = perm; b.inv = inv; b.scan_tmp = scan_tmp;
     b.nn = nn; b.nbr = nbr; b.flags = flags;
     b.bonds_on = bonds_on ? 1 : 0;
@@ -475,11 +477,13 @@ struct dem_ctx {
     if (kb[nsys] > (1l << 30)) return fail(DEM_ERR_ARG, "the binning grids need more than 2^30 cells in total");
     hipError_t e = hipStreamSynchronize(stream);
     if (e == hipSuccess && kb[nsys] > ncell_cap) {
-      hipFree(cell_count); hipFree(cell_start); hipFree(scan_tmp);
-      cell_count = cell_start = scan_tmp = nullptr;
+      hipFree(cell_count); hipFree(cell_scan); hipFree(cell_start); hipFree(scan_tmp);
+      cell_count = cell_scan = cell_start = scan_tmp = nullptr;
       cell_count = dalloc<int>((size_t)kb[nsys], &e);
+      cell_scan = dalloc<int>((size_t)kb[nsys], &e);
       cell_start = dalloc<int>((size_t)kb[nsys] + 1, &e);
       scan_tmp = dalloc<int>((size_t)(kb[nsys] / 4096 + 2), &e);
+      if (e == hipSuccess) e = hipMemset(cell_count, 0, (size_t)kb[nsys] * sizeof(int));
       if (e == hipSuccess) ncell_cap = kb[nsys];
     }
     if (e == hipSuccess && nsys > 1) {
@@ -634,12 +638,13 @@ struct dem_ctx {
   int rebuild(bool sync_check, bool check_skin, bool permute_ft = true) {
     mark_begin(1);
     BuildArgs b = build_args(check_skin && built_once, permute_ft);
-    hipError_t e = launch_rebuild(b, stream);
+    const bool small = rebuild_is_small(n, ncell);
+    hipError_t e = small ? launch_rebuild_small(b, stream) : launch_rebuild(b, stream);
     if (e != hipSuccess) return hip_fail(e, "rebuild launch");
     cP ^= 1; cS ^= 1; cC ^= 1;
     b = build_args(false);
     b.xr_out = xr[cP];
-    if ((e = launch_neighbors(b, stream)) != hipSuccess) return hip_fail(e, "neighbour launch");
+    if (!small && (e = launch_neighbors(b, stream)) != hipSuccess) return hip_fail(e, "neighbour launch");
     mark_end();
     built_once = true;
     list_valid = true;
@@ -896,6 +901,7 @@ int create_ctx(const dem_config* common, int nsys, const dem_system_desc* sd, de
   c->rank = dalloc<int>(n, &e);
   c->key_sorted = dalloc<int>(n, &e);
   c->cell_count = dalloc<int>((size_t)c->ncell, &e);
+  c->cell_scan = dalloc<int>((size_t)c->ncell, &e);
   c->cell_start = dalloc<int>((size_t)c->ncell + 1, &e);
   c->perm = dalloc<int>(n, &e);
   c->inv = dalloc<int>(n, &e);
@@ -934,6 +940,7 @@ int create_ctx(const dem_config* common, int nsys, const dem_system_desc* sd, de
   if (e == hipSuccess) e = hipMemset(c->xr[0], 0, n * sizeof(double4));
   if (e == hipSuccess) e = hipMemset(c->nn, 0, n * sizeof(int));
   if (e == hipSuccess) e = hipMemset(c->flags, 0, sizeof(DevFlags));
+  if (e == hipSuccess) e = hipMemset(c->cell_count, 0, (size_t)c->ncell * sizeof(int));
   for (int b = 0; b < 3; ++b) {
     if (e == hipSuccess)
       e = hipMemcpy(c->d_tile0_b[b], c->tile0_b[b].data(), (nsys + 1) * sizeof(int), hipMemcpyHostToDevice);

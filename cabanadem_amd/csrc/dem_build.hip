@@ -7,16 +7,20 @@
 // multiply-adds, exactly as the reference's Cabana build forms it, so the
 // sets are bit-exact.
 //
-// Sequence (one rebuild, all stream ordered):
+// Sequence (one rebuild, all stream ordered; small systems run all of it in
+// one workgroup, k_rebuild_small):
 //   1. k_cell_keys   cell key of every particle (tiled cell order, see
 //                    dem_internal.h); per-cell arrival rank by atomic
 //                    counting; optional skin-displacement check
-//   2. scan          exclusive prefix over the cell counts -> cell starts
+//   2. scan          exclusive prefix over the cell counts within scan tiles,
+//                    then over the tiles; clears the counts for the next
+//                    rebuild
 //   3. k_scatter     counting-sort scatter: slot = start[key] + rank
 //   4. k_cell_order  within each cell, order by previous slot (the arrival
 //                    order of step 1 is not deterministic; this makes the
 //                    sort a stable, deterministic single-digit radix sort
-//                    on the cell key) and write the inverse permutation
+//                    on the cell key), write the inverse permutation and the
+//                    cells' starts
 //   5. k_permute     gather the particle state into the new order and
 //                    re-map the tracked-contact lists (j -> inv[j], re-sorted)
 //   6. k_neighbors   27-cell search: for each (dz, dy) the three x-adjacent
@@ -38,10 +42,25 @@ __device__ inline int cell_coord(double v, const Grid& g, int d) {
   return (int)t;
 }
 
-__global__ __launch_bounds__(kBlock) void k_fill_int(int* p, long count, int value) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long stride = (long)gridDim.x * blockDim.x;
-  for (; i < count; i += stride) p[i] = value;
+// Cell key of slot i at position p; flags a position that is not finite.
+__device__ __forceinline__ int key_of(const BuildArgs& a, int i, const double4& p) {
+  if (!(isfinite(p.x) && isfinite(p.y) && isfinite(p.z))) atomicOr(&a.flags->nonfinite, 1);
+  // ensembles: the slot's system gives the grid and the first key
+  const int sys = a.sysid ? a.sysid[i] : 0;
+  const Grid& g = a.sysid ? a.grids[sys] : a.grid;
+  const long base = a.sysid ? a.kbase[sys] : 0;
+  const int cx = cell_coord(p.x, g, 0);
+  const int cy = cell_coord(p.y, g, 1);
+  const int cz = cell_coord(p.z, g, 2);
+  return (int)(base + cell_key(g, cx, cy, cz));
+}
+
+// Flags slot i when it has moved more than skin/2 since the last build.
+__device__ __forceinline__ void check_skin(const BuildArgs& a, int i, const double4& p) {
+  const double d0 = p.x - a.xb[3 * i + 0];
+  const double d1 = p.y - a.xb[3 * i + 1];
+  const double d2 = p.z - a.xb[3 * i + 2];
+  if (d0 * d0 + d1 * d1 + d2 * d2 > a.skin_half_sq) atomicOr(&a.flags->skin, 1);
 }
 
 // Per-cell arrival ranks with one atomic per run of equal keys in a wave:
@@ -57,15 +76,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_keys(BuildArgs a) {
   double4 p = make_double4(0., 0., 0., 0.);
   if (active) {
     p = a.xr_in[i];
-    if (!(isfinite(p.x) && isfinite(p.y) && isfinite(p.z))) atomicOr(&a.flags->nonfinite, 1);
-    // ensembles: the slot's system gives the grid and the first key
-    const int sys = a.sysid ? a.sysid[i] : 0;
-    const Grid& g = a.sysid ? a.grids[sys] : a.grid;
-    const long base = a.sysid ? a.kbase[sys] : 0;
-    const int cx = cell_coord(p.x, g, 0);
-    const int cy = cell_coord(p.y, g, 1);
-    const int cz = cell_coord(p.z, g, 2);
-    key = (int)(base + cell_key(g, cx, cy, cz));
+    key = key_of(a, i, p);
   }
   const int prev = __shfl_up(key, 1);
   const bool head = active && (lane == 0 || prev != key);
@@ -83,15 +94,10 @@ __global__ __launch_bounds__(kBlock) void k_cell_keys(BuildArgs a) {
   if (!active) return;
   a.key[i] = key;
   a.rank[i] = base_rank + (lane - hl);
-  if (a.check_skin) {
-    const double d0 = p.x - a.xb[3 * i + 0];
-    const double d1 = p.y - a.xb[3 * i + 1];
-    const double d2 = p.z - a.xb[3 * i + 2];
-    if (d0 * d0 + d1 * d1 + d2 * d2 > a.skin_half_sq) atomicOr(&a.flags->skin, 1);
-  }
+  if (a.check_skin) check_skin(a, i, p);
 }
 
-// ---- exclusive scan of int counts (three launches) -------------------------
+// ---- exclusive scan of the cell counts --------------------------------------
 constexpr int kScanThreads = 1024;
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanThreads * kScanItems;
@@ -112,7 +118,8 @@ __device__ inline int block_exclusive_scan(int v, int* lds, int* total) {
   return incl - v;
 }
 
-__global__ __launch_bounds__(kScanThreads) void k_scan_tiles(const int* in, int* out,
+// Also clears `in` (the next rebuild counts into it).
+__global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int* in, int* out,
                                                               int* tile_sums, long count) {
   __shared__ int lds[kScanThreads];
   const long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
@@ -127,14 +134,17 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(const int* in, int*
   int ex = block_exclusive_scan(s, lds, &total);
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
-    if (base + k < count) out[base + k] = ex;
+    if (base + k < count) {
+      out[base + k] = ex;
+      in[base + k] = 0;
+    }
     ex += v[k];
   }
   if (threadIdx.x == 0) tile_sums[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(kScanThreads) void k_scan_top(int* tile_sums, int ntiles,
-                                                            int* out, long count) {
+// Tile totals to tile offsets, and the build's longest row back to none.
+__global__ __launch_bounds__(kScanThreads) void k_scan_top(int* tile_sums, int ntiles, DevFlags* flags) {
   __shared__ int lds[kScanThreads];
   int carry = 0;
   for (int base = 0; base < ntiles; base += kScanThreads) {
@@ -145,35 +155,31 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_top(int* tile_sums, int n
     if (t < ntiles) tile_sums[t] = ex + carry;
     carry += total;
   }
-  if (threadIdx.x == 0) out[count] = carry;
+  if (threadIdx.x == 0) flags->max_nn = 0;
 }
 
-__global__ __launch_bounds__(kBlock) void k_scan_add(int* out, const int* tile_sums, long count) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count) out[i] += tile_sums[i / kScanTile];
-}
-
-hipError_t exclusive_scan(const int* in, int* out, int* tmp, long count, hipStream_t s) {
-  const int ntiles = (int)((count + kScanTile - 1) / kScanTile);
-  hipLaunchKernelGGL(k_scan_tiles, dim3(ntiles), dim3(kScanThreads), 0, s, in, out, tmp, count);
-  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanThreads), 0, s, tmp, ntiles, out, count);
-  hipLaunchKernelGGL(k_scan_add, dim3((unsigned)((count + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                     s, out, tmp, count);
-  return hipGetLastError();
+// Start of cell c: its place in its scan tile on top of the tile's offset
+// (added by the two readers instead of a pass over all cells).
+__device__ __forceinline__ int start_of(const BuildArgs& a, long c) {
+  return c < a.ncell ? a.cell_scan[c] + a.scan_tmp[c / kScanTile] : a.n;
 }
 
 __global__ __launch_bounds__(kBlock) void k_scatter(BuildArgs a) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= a.n) return;
-  a.perm[a.cell_start[a.key[i]] + a.rank[i]] = i;
+  a.perm[start_of(a, a.key[i]) + a.rank[i]] = i;
 }
 
 // One thread per cell: insertion-sort the cell's slots by previous index
-// (cells hold a handful of particles), then record old -> new.
+// (cells hold a handful of particles), then record old -> new and the cell's
+// start.
 __global__ __launch_bounds__(kBlock) void k_cell_order(BuildArgs a) {
   const long c = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (c >= a.ncell) return;
-  const int s = a.cell_start[c], e = a.cell_start[c + 1];
+  if (c > a.ncell) return;
+  const int s = start_of(a, c);
+  a.cell_start[c] = s;
+  if (c == a.ncell) return;
+  const int e = start_of(a, c + 1);
   if (e - s > kMaxCellParticles) {
     atomicOr(&a.flags->cell_overflow, 1);
     for (int q = s; q < e; ++q) a.inv[a.perm[q]] = q;
@@ -191,6 +197,13 @@ __global__ __launch_bounds__(kBlock) void k_cell_order(BuildArgs a) {
   for (int q = s; q < e; ++q) a.inv[a.perm[q]] = q;
 }
 
+// A wave's own LDS tile: its writes before its later reads, and back.
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ inline void copy6(const double* src, double* dst) {
   const double2* s = reinterpret_cast<const double2*>(src);
   double2* d = reinterpret_cast<double2*>(dst);
@@ -199,29 +212,10 @@ __device__ inline void copy6(const double* src, double* dst) {
   d[2] = s[2];
 }
 
-// Gather the per-particle arrays into the new order.  The tracked-contact
-// list of a particle keeps its entries and histories; only the neighbour
-// indices change (j -> inv[j]) and the list is re-sorted by the new index.
-__global__ __launch_bounds__(kBlock) void k_permute(BuildArgs a) {
-  extern __shared__ int s_j[]; // [max_c][kBlock]
-  const int tid = threadIdx.x;
-  const int p = blockIdx.x * kBlock + tid;
-  if (p >= a.n) return;
-  const int o = a.perm[p];
-  const double4 xr = a.xr_in[o];
-  a.xr_out[p] = xr;
-  copy6(a.uw_in + 6l * o, a.uw_out + 6l * p);
-  if (a.permute_ft) copy6(a.ft_in + 6l * o, a.ft_out + 6l * p);
-  a.mat_out[p] = a.mat_in[o];
-  a.mI_out[p] = a.mI_in[o];
-  a.id_out[p] = a.id_in[o];
-  a.key_sorted[p] = a.key[o];
-  if (a.keep_xb) {
-    a.xb[3 * p + 0] = xr.x;
-    a.xb[3 * p + 1] = xr.y;
-    a.xb[3 * p + 2] = xr.z;
-  }
-  const int meta = a.cmeta_in[o];
+// Slot p's particle (old slot o): contact word, wall histories, bonds, group and
+// external force.  inv(j): the new slot of old slot j.
+template <class Inv>
+__device__ __forceinline__ void permute_lists(const BuildArgs& a, int p, int o, int meta, const Inv& inv) {
   a.cmeta_out[p] = meta;
   const int wm = meta_walls(meta);
   if (wm) {
@@ -238,7 +232,7 @@ __global__ __launch_bounds__(kBlock) void k_permute(BuildArgs a) {
     if (a.vgroup_in) a.vgroup_out[p] = a.vgroup_in[o];
     for (int b = 0; b < nb; ++b) {
       const int j = a.bj_in[(long)b * a.ld + o];
-      a.bj_out[(long)b * a.ld + p] = j >= 0 ? a.inv[j] : -1;
+      a.bj_out[(long)b * a.ld + p] = j >= 0 ? inv(j) : -1;
       a.bl_out[(long)b * a.ld + p] = a.bl_in[(long)b * a.ld + o];
       for (int c = 0; c < 9; ++c)
         a.bh_out[(long)(9 * b + c) * a.ld + p] = a.bh_in[(long)(9 * b + c) * a.ld + o];
@@ -248,40 +242,186 @@ __global__ __launch_bounds__(kBlock) void k_permute(BuildArgs a) {
   }
   if (a.fext_in)
     for (int d = 0; d < 3; ++d) a.fext_out[3l * p + d] = a.fext_in[3l * o + d];
-  int oc = meta_count(meta);
-  if (oc > a.max_c) oc = a.max_c; // counts are clamped on write; never index past the LDS rows
-  for (int m = 0; m < oc; ++m) s_j[m * kBlock + tid] = a.inv[a.cj_in[(long)m * a.ld + o]];
+}
+
+// The tracked-contact list of a particle keeps its entries and histories; only
+// the neighbour indices change (old j -> its new slot, id(m) for entry m) and
+// the list is re-sorted by the new index.
+template <class Id>
+__device__ __forceinline__ void permute_contacts(const BuildArgs& a, int p, int o, int oc, const Id& id) {
   for (int m = 0; m < oc; ++m) {
-    const int jm = s_j[m * kBlock + tid];
+    const int jm = id(m);
     int r = 0;
-    for (int q = 0; q < oc; ++q) r += (s_j[q * kBlock + tid] < jm) ? 1 : 0;
+    for (int q = 0; q < oc; ++q) r += (id(q) < jm) ? 1 : 0;
     a.cj_out[(long)r * a.ld + p] = jm;
     for (int c = 0; c < 3; ++c)
       a.ch_out[(long)(r * 3 + c) * a.ld + p] = a.ch_in[(long)(m * 3 + c) * a.ld + o];
   }
 }
 
-__device__ inline int wave_max_int(int v) {
-  for (int off = 32; off > 0; off >>= 1) {
-    const int o = __shfl_xor(v, off);
-    v = o > v ? o : v;
+__device__ __forceinline__ void permute_state(const BuildArgs& a, int p, int o, const double4& xr) {
+  a.xr_out[p] = xr;
+  copy6(a.uw_in + 6l * o, a.uw_out + 6l * p);
+  if (a.permute_ft) copy6(a.ft_in + 6l * o, a.ft_out + 6l * p);
+  a.mat_out[p] = a.mat_in[o];
+  a.mI_out[p] = a.mI_in[o];
+  a.id_out[p] = a.id_in[o];
+  if (a.keep_xb) {
+    a.xb[3 * p + 0] = xr.x;
+    a.xb[3 * p + 1] = xr.y;
+    a.xb[3 * p + 2] = xr.z;
   }
-  return v;
 }
 
-__device__ inline int wave_min_int(int v) {
-  for (int off = 32; off > 0; off >>= 1) {
-    const int o = __shfl_xor(v, off);
-    v = o < v ? o : v;
+// A wave's consecutive records from its LDS tile to memory, 16 bytes a lane and
+// instruction on consecutive addresses (past the caches with nt): n16 pieces.
+template <int K>
+__device__ __forceinline__ void store_records(const double2* st, double2* g, int n16, int lane, bool nt) {
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int q = k * 64 + lane;
+    if (q >= n16) continue;
+    const double2 v = st[q];
+    if (nt) {
+      __builtin_nontemporal_store(v.x, &g[q].x);
+      __builtin_nontemporal_store(v.y, &g[q].y);
+    } else {
+      g[q] = v;
+    }
   }
-  return v;
 }
 
-// A wave's own LDS tile: its writes before its later reads, and back.
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// Gather the per-particle arrays into the new order.  Everything of the
+// particle is loaded before anything is stored (a store in between would wait
+// for the load before it, and no load moves up over a store), and the records
+// leave through LDS in whole lines, as in the fused step.  Bound: HBM, about
+// 310 bytes a particle.  1M spheres 75 -> 66 us (4.7 TB/s), 4M 270 -> 232.
+__global__ __launch_bounds__(kBlock) void k_permute(BuildArgs a) {
+  extern __shared__ int s_j[]; // [max_c][kBlock]
+  __shared__ double2 s_rec[kBlock / 64][64 * 5];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int p0 = blockIdx.x * kBlock + tid - lane; // the wave's first slot
+  const int cnt = min(64, a.n - p0);
+  const int p = p0 + lane;
+  const bool act = p < a.n;
+  double2* st = s_rec[tid >> 6];
+  const bool nt = a.stream != 0;
+  double* sx = reinterpret_cast<double*>(st + 128);
+  double4 xr, mat;
+  double2 u0, u1, u2, mI;
+  int o = 0, id = 0, key = 0, meta = 0, oc = 0;
+  if (act) {
+    o = a.perm[p];
+    xr = a.xr_in[o];
+    const double2* uo = reinterpret_cast<const double2*>(a.uw_in + 6l * o);
+    u0 = uo[0]; u1 = uo[1]; u2 = uo[2];
+    mat = a.mat_in[o];
+    mI = a.mI_in[o];
+    id = a.id_in[o];
+    key = a.key[o];
+    meta = a.cmeta_in[o];
+    oc = min(meta_count(meta), a.max_c); // counts are clamped on write; never index past the LDS rows
+    for (int m = 0; m < oc; ++m) s_j[m * kBlock + tid] = a.inv[a.cj_in[(long)m * a.ld + o]];
+    st[2 * lane] = make_double2(xr.x, xr.y);
+    st[2 * lane + 1] = make_double2(xr.z, xr.w);
+    st[128 + 3 * lane] = u0;
+    st[128 + 3 * lane + 1] = u1;
+    st[128 + 3 * lane + 2] = u2;
+  }
+  wave_lds_sync();
+  store_records<2>(st, reinterpret_cast<double2*>(a.xr_out + p0), 2 * cnt, lane, false);
+  store_records<3>(st + 128, reinterpret_cast<double2*>(a.uw_out + 6l * p0), 3 * cnt, lane, nt);
+  wave_lds_sync();
+  if (act) {
+    st[2 * lane] = make_double2(mat.x, mat.y);
+    st[2 * lane + 1] = make_double2(mat.z, mat.w);
+    sx[3 * lane] = xr.x;
+    sx[3 * lane + 1] = xr.y;
+    sx[3 * lane + 2] = xr.z;
+  }
+  wave_lds_sync();
+  store_records<2>(st, reinterpret_cast<double2*>(a.mat_out + p0), 2 * cnt, lane, nt);
+  if (a.keep_xb) {
+    double* xb = a.xb + 3l * p0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (k * 64 + lane < 3 * cnt) xb[k * 64 + lane] = sx[k * 64 + lane];
+  }
+  if (!act) return;
+  a.mI_out[p] = mI;
+  a.id_out[p] = id;
+  a.key_sorted[p] = key;
+  if (a.permute_ft) copy6(a.ft_in + 6l * o, a.ft_out + 6l * p);
+  permute_lists(a, p, o, meta, [&](int j) { return a.inv[j]; });
+  permute_contacts(a, p, o, oc, [&](int m) { return s_j[m * kBlock + tid]; });
+}
+
+// Minimum and maximum over the wave's 64 lanes, the same scalar in all of
+// them: row shifts and row broadcasts in the VALU, where shuffles go through
+// LDS six times over, each waiting for the one before (k_neighbors at 1M
+// spheres, eighteen reductions a wave: 71 -> 68 us).  Every lane of the wave
+// must call these.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_or(int fill, int v) {
+  return __builtin_amdgcn_update_dpp(fill, v, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ int wave_max_int(int v) {
+  v = max(v, dpp_or<0x111, 0xf>(INT_MIN, v)); // row_shr 1, 2, 4, 8: lane 15 of a row holds the row's
+  v = max(v, dpp_or<0x112, 0xf>(INT_MIN, v));
+  v = max(v, dpp_or<0x114, 0xf>(INT_MIN, v));
+  v = max(v, dpp_or<0x118, 0xf>(INT_MIN, v));
+  v = max(v, dpp_or<0x142, 0xa>(INT_MIN, v)); // row_bcast 15 into rows 1 and 3
+  v = max(v, dpp_or<0x143, 0xc>(INT_MIN, v)); // row_bcast 31 into rows 2 and 3
+  return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ int wave_min_int(int v) {
+  v = min(v, dpp_or<0x111, 0xf>(INT_MAX, v));
+  v = min(v, dpp_or<0x112, 0xf>(INT_MAX, v));
+  v = min(v, dpp_or<0x114, 0xf>(INT_MAX, v));
+  v = min(v, dpp_or<0x118, 0xf>(INT_MAX, v));
+  v = min(v, dpp_or<0x142, 0xa>(INT_MAX, v));
+  v = min(v, dpp_or<0x143, 0xc>(INT_MAX, v));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// The nine slot ranges around slot p's cell `key`: three consecutive x-cells of
+// one (y, z) row each, ascending by start (they never overlap), INT_MAX where
+// there is none.  start(c): first slot of cell c.
+template <class Start>
+__device__ __forceinline__ void slot_ranges(const BuildArgs& a, int p, int key, const Start& start, int (&rs)[9],
+                                            int (&re)[9]) {
+  const int sys = a.sysid ? a.sysid[p] : 0;
+  const Grid& g = a.sysid ? a.grids[sys] : a.grid;
+  const long base = a.sysid ? a.kbase[sys] : 0;
+  const int nx = g.nc[0], ny = g.nc[1], nz = g.nc[2];
+  key = (int)(key - base);
+  const int cx = key % nx;
+  key /= nx;
+  const int ly = key % g.tr;
+  key /= g.tr;
+  const int cz = key % nz;
+  const int cy = (key / nz) * g.tr + ly;
+  const int xlo = cx > 0 ? cx - 1 : 0;
+  const int xhi = cx < nx - 1 ? cx + 1 : nx - 1;
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    const int z = cz + q / 3 - 1, y = cy + q % 3 - 1;
+    const bool in = z >= 0 && z < nz && y >= 0 && y < ny;
+    rs[q] = re[q] = INT_MAX;
+    if (in) {
+      const long k0 = base + cell_key(g, xlo, y, z);
+      rs[q] = start(k0);
+      re[q] = start(k0 + (xhi - xlo) + 1);
+    }
+  }
+#pragma unroll
+  for (int q = 1; q < 9; ++q)
+#pragma unroll
+    for (int r = q; r > 0; --r)
+      if (rs[r] < rs[r - 1]) {
+        int t = rs[r]; rs[r] = rs[r - 1]; rs[r - 1] = t;
+        t = re[r]; re[r] = re[r - 1]; re[r - 1] = t;
+      }
 }
 
 #ifndef DEM_NBR_STAGE
@@ -317,38 +457,8 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(BuildArgs a) {
     re[q] = INT_MAX;
   }
   if (active) {
-    const int sys = a.sysid ? a.sysid[p] : 0;
-    const Grid& g = a.sysid ? a.grids[sys] : a.grid;
-    const long base = a.sysid ? a.kbase[sys] : 0;
-    const int nx = g.nc[0], ny = g.nc[1], nz = g.nc[2];
-    int key = (int)(a.key_sorted[p] - base);
-    const int cx = key % nx;
-    key /= nx;
-    const int ly = key % g.tr;
-    key /= g.tr;
-    const int cz = key % nz;
-    const int cy = (key / nz) * g.tr + ly;
     xi = a.xr_out[p];
-    const int xlo = cx > 0 ? cx - 1 : 0;
-    const int xhi = cx < nx - 1 ? cx + 1 : nx - 1;
-    // the nine slot ranges, ascending by start (they never overlap)
-#pragma unroll
-    for (int q = 0; q < 9; ++q) {
-      const int z = cz + q / 3 - 1, y = cy + q % 3 - 1;
-      if (z >= 0 && z < nz && y >= 0 && y < ny) {
-        const long k0 = base + cell_key(g, xlo, y, z);
-        rs[q] = a.cell_start[k0];
-        re[q] = a.cell_start[k0 + (xhi - xlo) + 1];
-      }
-    }
-#pragma unroll
-    for (int q = 1; q < 9; ++q)
-#pragma unroll
-      for (int r = q; r > 0; --r)
-        if (rs[r] < rs[r - 1]) {
-          int t = rs[r]; rs[r] = rs[r - 1]; rs[r - 1] = t;
-          t = re[r]; re[r] = re[r - 1]; re[r - 1] = t;
-        }
+    slot_ranges(a, p, a.key_sorted[p], [&](long c) { return a.cell_start[c]; }, rs, re);
   }
 #pragma unroll
   for (int q = 0; q < 9; ++q) {
@@ -357,29 +467,28 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(BuildArgs a) {
     const int lo = wave_min_int(has ? s : INT_MAX);
     const int hi = wave_max_int(has ? e : INT_MIN);
     if (lo == INT_MAX) break; // no lane has a q-th range, nor a later one
-    // the same for the whole wave; readfirstlane lets the compiler branch on it
-    const bool staged = __builtin_amdgcn_readfirstlane(hi - lo <= kNbrStage ? 1 : 0) != 0;
-    auto test = [&](int j, const double4& xj) {
+    const bool staged = hi - lo <= kNbrStage; // the same for the whole wave
+    const auto within = [&](const double4& xj) {
       const double d0 = xi.x - xj.x;
       const double d1 = xi.y - xj.y;
       const double d2 = xi.z - xj.z;
-      const double dsqr = d0 * d0 + d1 * d1 + d2 * d2;
-      if (dsqr <= a.rc2) {
-        if (cnt < a.max_n) a.nbr[off] = j;
-        ++cnt;
-        off += a.ld;
-      }
+      return d0 * d0 + d1 * d1 + d2 * d2 <= a.rc2;
+    };
+    const auto add = [&](int j) {
+      if (cnt < a.max_n) a.nbr[off] = j;
+      ++cnt;
+      off += a.ld;
     };
     if (staged) {
       for (int t = lane; t < hi - lo; t += 64) sx[w][t] = a.xr_out[lo + t];
       wave_lds_sync();
       if (has)
         for (int j = s; j < e; ++j)
-          if (j != p) test(j, sx[w][j - lo]);
+          if (j != p && within(sx[w][j - lo])) add(j);
       wave_lds_sync(); // the next round rewrites the tile
     } else if (has) {
       for (int j = s; j < e; ++j)
-        if (j != p) test(j, a.xr_out[j]);
+        if (j != p && within(a.xr_out[j])) add(j);
     }
   }
   if (active) a.nn[p] = cnt < a.max_n ? cnt : a.max_n;
@@ -388,6 +497,120 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(BuildArgs a) {
   if (lane == 0 && wmax > 0) {
     if (wmax > *(volatile int*)&a.flags->max_nn) atomicMax(&a.flags->max_nn, wmax);
     if (wmax > a.max_n) atomicMax(&a.flags->nbr_overflow, wmax);
+  }
+}
+
+// The whole rebuild of a small system in one workgroup: the sequence above with
+// the counts, the sort and the positions in LDS and barriers for launches.  A
+// rebuild of eight launches costs a small system 30 us and more, launch gaps
+// for the most part, and by default it comes every step.
+constexpr int kSmallThreads = 1024;
+// Rebuilt every step, us a step with eight launches / one workgroup: 2 spheres
+// 37 / 14, 64 47 / 25, 512 58 / 40, 1,000 60 / 50, 1,728 61 / 78.
+constexpr int kSmallMax = 1024;        // particles
+constexpr int kSmallCells = 8192;      // cells, all systems
+
+__global__ __launch_bounds__(kSmallThreads) void k_rebuild_small(BuildArgs a) {
+  __shared__ double4 pos[kSmallMax];      // new order
+  __shared__ int start[kSmallCells + 1];  // counts, then starts
+  __shared__ int perm[kSmallMax], inv[kSmallMax], key[kSmallMax];
+  __shared__ int wsum[kSmallThreads / 64];
+  const int tid = threadIdx.x, T = blockDim.x, lane = tid & 63, w = tid >> 6;
+  const int ncell = (int)a.ncell;
+  for (int c = tid; c <= ncell; c += T) start[c] = 0;
+  __syncthreads();
+  static_assert(kSmallMax <= kSmallThreads, "a thread per particle");
+  int rank = 0;
+  if (tid < a.n) {
+    const double4 p = a.xr_in[tid];
+    key[tid] = key_of(a, tid, p);
+    rank = atomicAdd(&start[key[tid]], 1);
+    if (a.check_skin) check_skin(a, tid, p);
+  }
+  __syncthreads();
+  { // counts -> starts: each thread a run of cells, then a scan over the threads
+    const int per = (ncell + T - 1) / T, c0 = tid * per, c1 = min(ncell, c0 + per);
+    int sum = 0;
+    for (int c = c0; c < c1; ++c) sum += start[c];
+    int incl = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+      const int t = __shfl_up(incl, off);
+      if (lane >= off) incl += t;
+    }
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    int run = incl - sum;
+    for (int k = 0; k < w; ++k) run += wsum[k];
+    for (int c = c0; c < c1; ++c) {
+      const int n = start[c];
+      start[c] = run;
+      run += n;
+    }
+    if (tid == 0) start[ncell] = a.n;
+  }
+  __syncthreads();
+  if (tid < a.n) perm[start[key[tid]] + rank] = tid;
+  __syncthreads();
+  for (int c = tid; c < ncell; c += T) { // within a cell by previous slot, as k_cell_order
+    const int s = start[c], e = start[c + 1];
+    for (int q = s + 1; q < e; ++q) {
+      const int v = perm[q];
+      int r = q - 1;
+      while (r >= s && perm[r] > v) {
+        perm[r + 1] = perm[r];
+        --r;
+      }
+      perm[r + 1] = v;
+    }
+    for (int q = s; q < e; ++q) inv[perm[q]] = q;
+  }
+  __syncthreads();
+  const int p = tid;
+  const int o = p < a.n ? perm[p] : 0;
+  if (p < a.n) {
+    const double4 xr = a.xr_in[o];
+    pos[p] = xr;
+    permute_state(a, p, o, xr);
+    a.key_sorted[p] = key[o];
+    const auto new_slot = [&](int j) { return inv[j]; };
+    const int meta = a.cmeta_in[o];
+    permute_lists(a, p, o, meta, new_slot);
+    permute_contacts(a, p, o, min(meta_count(meta), a.max_c), [&](int m) { return inv[a.cj_in[(long)m * a.ld + o]]; });
+  }
+  __syncthreads();
+  int longest = 0;
+  if (p < a.n) {
+    int rs[9], re[9];
+    slot_ranges(a, p, key[o], [&](long c) { return start[c]; }, rs, re);
+    const double4 xi = pos[p];
+    int cnt = 0;
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+      if (rs[q] == INT_MAX) break;
+      for (int j = rs[q]; j < re[q]; ++j) {
+        const double4 xj = pos[j];
+        const double d0 = xi.x - xj.x;
+        const double d1 = xi.y - xj.y;
+        const double d2 = xi.z - xj.z;
+        const double dsqr = d0 * d0 + d1 * d1 + d2 * d2;
+        if (j != p && dsqr <= a.rc2) {
+          if (cnt < a.max_n) a.nbr[(long)cnt * a.ld + p] = j;
+          ++cnt;
+        }
+      }
+    }
+    a.nn[p] = cnt < a.max_n ? cnt : a.max_n;
+    longest = cnt;
+  }
+  longest = wave_max_int(longest);
+  if (lane == 0) wsum[w] = longest;
+  __syncthreads();
+  for (int k = 0; k < T / 64; ++k) longest = max(longest, wsum[k]);
+  if (longest > a.max_n) // the caller searches again with longer rows: k_neighbors needs the starts
+    for (int c = tid; c <= ncell; c += T) a.cell_start[c] = start[c];
+  if (tid == 0) {
+    a.flags->max_nn = longest;
+    if (longest > a.max_n) atomicMax(&a.flags->nbr_overflow, longest);
   }
 }
 
@@ -438,24 +661,24 @@ hipError_t launch_setup_bonds(const BondSetupArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_fill_int(int* p, long count, int value, hipStream_t s) {
-  if (count <= 0) return hipSuccess;
-  long blocks = (count + kBlock - 1) / kBlock;
-  if (blocks > 65535L * 8) blocks = 65535L * 8;
-  hipLaunchKernelGGL(k_fill_int, dim3((unsigned)blocks), dim3(kBlock), 0, s, p, count, value);
+bool rebuild_is_small(int n, long ncell) { return n <= kSmallMax && ncell <= kSmallCells; }
+
+hipError_t launch_rebuild_small(const BuildArgs& a, hipStream_t s) {
+  // a thread per particle, and enough of them for the cells
+  const long want = std::max<long>(a.n, a.ncell / 16);
+  const int threads = (int)std::min<long>(kSmallThreads, (want + 63) / 64 * 64);
+  hipLaunchKernelGGL(k_rebuild_small, dim3(1), dim3(threads), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_rebuild(const BuildArgs& a, hipStream_t s) {
-  hipError_t e = launch_fill_int(&a.flags->max_nn, 1, 0, s);
-  if (e != hipSuccess) return e;
-  e = launch_fill_int(a.cell_count, a.ncell, 0, s);
-  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_cell_keys, dim3(nblk(a.n)), dim3(kBlock), 0, s, a);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = exclusive_scan(a.cell_count, a.cell_start, a.scan_tmp, a.ncell, s)) != hipSuccess) return e;
+  const int ntiles = (int)((a.ncell + kScanTile - 1) / kScanTile);
+  hipLaunchKernelGGL(k_scan_tiles, dim3(ntiles), dim3(kScanThreads), 0, s, a.cell_count, a.cell_scan, a.scan_tmp,
+                     a.ncell);
+  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanThreads), 0, s, a.scan_tmp, ntiles, a.flags);
   hipLaunchKernelGGL(k_scatter, dim3(nblk(a.n)), dim3(kBlock), 0, s, a);
-  hipLaunchKernelGGL(k_cell_order, dim3(nblk(a.ncell)), dim3(kBlock), 0, s, a);
+  hipLaunchKernelGGL(k_cell_order, dim3(nblk(a.ncell + 1)), dim3(kBlock), 0, s, a);
   const size_t lds = (size_t)(a.max_c > 0 ? a.max_c : 1) * kBlock * sizeof(int);
   hipLaunchKernelGGL(k_permute, dim3(nblk(a.n)), dim3(kBlock), lds, s, a);
   return hipGetLastError();

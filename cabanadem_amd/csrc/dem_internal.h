@@ -228,6 +228,7 @@ struct BuildArgs {
   int check_skin;    // compare with the positions of the last build
   int keep_xb;       // record the positions of this build
   int permute_ft;    // F and T are live across this rebuild
+  int stream;        // as StepArgs::stream
   // old (cur) and new (nxt) buffers
   const double4* xr_in; double4* xr_out;
   const double* uw_in; double* uw_out;
@@ -243,7 +244,8 @@ struct BuildArgs {
   int* key;     // cell key, old order
   int* rank;    // arrival rank in the cell, old order
   int* key_sorted;
-  int* cell_count;
+  int* cell_count; // zero between rebuilds
+  int* cell_scan;  // starts within the scan tiles
   int* cell_start;
   int* perm;    // new -> old
   int* inv;     // old -> new
@@ -280,7 +282,10 @@ hipError_t launch_setup_bonds(const BondSetupArgs& a, hipStream_t s);
 // Launchers (defined in dem_build.hip / dem_force.hip); all enqueue on `s`.
 hipError_t launch_rebuild(const BuildArgs& a, hipStream_t s);
 hipError_t launch_neighbors(const BuildArgs& a, hipStream_t s);
-hipError_t launch_fill_int(int* p, long count, int value, hipStream_t s);
+// launch_rebuild and launch_neighbors (over the buffers as launch_rebuild
+// writes them) in one launch, for systems that fit one workgroup.
+bool rebuild_is_small(int n, long ncell);
+hipError_t launch_rebuild_small(const BuildArgs& a, hipStream_t s);
 // p[0 .. count) = 0 (count <= 64)
 hipError_t launch_zero_u64(unsigned long long* p, int count, hipStream_t s);
 
