@@ -1605,11 +1605,21 @@ int launch_edge(const EdgeFwdArgs& a, int grid_cap, void* stream) {
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-// Rows of a chunk of the parameter gradients, at least.
-#ifndef GNN_GRAD_ROWS
-#define GNN_GRAD_ROWS 512
-#endif
-constexpr int kGradRows = GNN_GRAD_ROWS;
+void launch_wgrad(const WgradPairArgs& g, bool narrow, bool wide, dim3 grid, hipStream_t s) {
+  const dim3 b(64 * kWgWaves);
+  const int dy = !wide ? kDyNarrow : !g.add ? kDyOnly : g.dY ? kDyAndAdd : kAddOnly;
+  if (narrow) {
+    if (dy == kDyNarrow) hipLaunchKernelGGL((k_wgrad_pair<false, kDyNarrow>), grid, b, 0, s, g);
+    else if (dy == kDyOnly) hipLaunchKernelGGL((k_wgrad_pair<false, kDyOnly>), grid, b, 0, s, g);
+    else if (dy == kAddOnly) hipLaunchKernelGGL((k_wgrad_pair<false, kAddOnly>), grid, b, 0, s, g);
+    else hipLaunchKernelGGL((k_wgrad_pair<false, kDyAndAdd>), grid, b, 0, s, g);
+  } else {
+    if (dy == kDyNarrow) hipLaunchKernelGGL((k_wgrad_pair<true, kDyNarrow>), grid, b, 0, s, g);
+    else if (dy == kDyOnly) hipLaunchKernelGGL((k_wgrad_pair<true, kDyOnly>), grid, b, 0, s, g);
+    else if (dy == kAddOnly) hipLaunchKernelGGL((k_wgrad_pair<true, kAddOnly>), grid, b, 0, s, g);
+    else hipLaunchKernelGGL((k_wgrad_pair<true, kDyAndAdd>), grid, b, 0, s, g);
+  }
+}
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -1723,8 +1733,8 @@ int gnn_weight_grad(const gnn_mlp_io* io, const void* G_bf16, const float* G_f32
 int gnn_mlp_grads(const gnn_mlp_io* io, const gnn_mlp_weights* wt, const float* dY, const float* add,
                   const int* add_idx, const void* hidden, float* const dX[3], int accumulate, void* dH,
                   void* dYb, float* work, long work_floats, float* grad, void* stream) {
-  if (check_io(io) || !wt || (!dY && !add) || (add && !add_idx) || !hidden || !dH || !dYb || !work || !grad ||
-      !wt->W1 || !wt->W2)
+  if (check_io(io) || !wt || (!dY && !add) || (add && !add_idx) || !hidden || !dH || !work || !grad ||
+      !wt->W2)
     return -1;
   const bool wide = wt->nout_pad == kLat && wt->nout == kLat;
   if (!wide && (wt->nout_pad != 16 || wt->nout < 1 || wt->nout > 16 || add || !dY)) return -1;
@@ -1752,51 +1762,47 @@ int gnn_mlp_grads(const gnn_mlp_io* io, const gnn_mlp_weights* wt, const float* 
   a.dH = reinterpret_cast<bf16*>(dH);
   a.dYb = reinterpret_cast<bf16*>(dYb);
   int nx = 0;
+  bool in_place = false;
   for (int q = 0; dX && q < io->nseg; ++q) {
     if (!dX[q]) continue;
     if (nx == 2 || narrow || !aligned16(dX[q])) return -1;
     a.W1[nx] = reinterpret_cast<const bf16*>(wt->W1) + (long)in.start[q] * kLat;
     a.dX[nx] = dX[q];
     // dY of the same rows is in registers when its gradient accumulates there
-    const bool acc = (accumulate >> q) & 1;
-    a.mode[nx] = !acc ? 0 : (wide && (dX[q] == dY || !dY) ? 2 : 1);
+    const bool acc = (accumulate >> q) & 1, residual = (accumulate >> (3 + q)) & 1;
+    if (residual && !wide) return -1;
+    a.mode[nx] = residual || (acc && wide && (dX[q] == dY || !dY)) ? 2 : acc;
+    in_place = in_place || dX[q] == dY;
     ++nx;
   }
   const long cw = (long)(K + 1) * kLat + (long)kLat * wt->nout_pad;
+  const int chunk = ((io->M + kGradChunks - 1) / kGradChunks + 31) / 32 * 32;
+  const int nch = (io->M + chunk - 1) / chunk;
+  if ((long)nch * (kBiasCols + cw) > work_floats) return -1;
   const int per = 16 * kBwdWaves;
   int grid = (io->M + per - 1) / per;
   if (grid > cus) grid = cus;
-  // chunks of the parameter gradients: one block per CU over all 128-wide
-  // blocks of columns, chunks a multiple of 8 (the blocks of one chunk then
-  // share an XCD's L2) and at least kGradRows rows each
-  const int nby = (narrow ? 1 : io->nseg) + 1;
-  int nch = cus / nby / 8 * 8;
-  const int most = (io->M + kGradRows - 1) / kGradRows;
-  if (nch < 1) nch = 1;
-  if (nch > most) nch = most;
-  const int step = 32 * kWgWaves;
-  const int chunk = ((io->M + nch - 1) / nch + step - 1) / step * step;
-  nch = (io->M + chunk - 1) / chunk;
-  if ((long)grid * kBiasCols + (long)nch * cw > work_floats) return -1;
-  a.bpart = work;
-  if (int r = wide ? launch_bwd_rows<kLat>(a, nx, grid, s) : launch_bwd_rows<16>(a, nx, grid, s)) return r;
   WgradPairArgs g{};
   g.M = io->M;
   g.K = K;
   g.NO = wt->nout_pad;
+  g.nout = wt->nout;
   g.chunk = chunk;
   g.in = in;
   g.dH = a.dH;
   g.hid = a.hid;
-  g.dYb = a.dYb;
-  g.part = work + (long)grid * kBiasCols;
-  const dim3 gg(nch, nby), gb(64 * kWgWaves);
-  if (narrow && wide) hipLaunchKernelGGL((k_wgrad_pair<2, 8>), gg, gb, 0, s, g);
-  else if (narrow) hipLaunchKernelGGL((k_wgrad_pair<2, 1>), gg, gb, 0, s, g);
-  else if (wide) hipLaunchKernelGGL((k_wgrad_pair<8, 8>), gg, gb, 0, s, g);
-  else hipLaunchKernelGGL((k_wgrad_pair<8, 1>), gg, gb, 0, s, g);
-  hipLaunchKernelGGL(k_grad_reduce, dim3((unsigned)(cw / kLat + 1)), dim3(kThreads), 0, s, (const float*)g.part, nch,
-                     (const float*)a.bpart, grid, K, wt->nout_pad, grad);
+  g.dY = dY;
+  g.add = add;
+  g.idx = add_idx;
+  g.bpart = work;
+  g.part = work + (long)nch * kBiasCols;
+  const int blocks_x = (nch + 7) / 8 * 8, rows_of_blocks = (narrow ? 1 : io->nseg) + 1;
+  // W2 reads dY: before k_bwd_rows where that overwrites it, else beside W1
+  if (in_place) launch_wgrad(g, narrow, wide, dim3(blocks_x, 1), s);
+  if (int r = wide ? launch_bwd_rows<kLat>(a, nx, grid, s) : launch_bwd_rows<16>(a, nx, grid, s)) return r;
+  g.y0 = in_place ? 1 : 0;
+  launch_wgrad(g, narrow, wide, dim3(blocks_x, rows_of_blocks - g.y0), s);
+  hipLaunchKernelGGL(k_grad_reduce, dim3(nblk(cw + wt->nout_pad)), dim3(kThreads), 0, s, (const float*)g.part, nch, (const float*)work, K, wt->nout_pad, grad);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

@@ -3,9 +3,9 @@
 // edge MLP's gradients at the nodes it gathered.
 //
 //   k_bwd_rows     dY' = dY + add[idx];  dH = (dY' W2^T) * [hid > 0];
-//                  dX = dH W1^T for up to two input sources; dY' in BF16 and
-//                  the FP32 column sums of dY' (db2)
-//   k_wgrad_pair   partial dW1 = X^T dH, db1 and dW2 = hid^T dY' over row chunks
+//                  dX = dH W1^T for up to two input sources
+//   k_wgrad_pair   partial dW2 = hid^T dY', db2, dW1 = X^T dH and db1 over row
+//                  chunks
 //   k_grad_reduce  the partials summed in chunk order into W1 | b1 | W2 | b2
 //   k_edge_hidden_to_nodes
 //                  dh[i] += sum over the edges e of i of dH[e] W1b^T
@@ -14,6 +14,7 @@
 
 constexpr int kBwdWaves = 8;
 constexpr int kBiasCols = kLat; // a partial row of db2
+constexpr int kGradChunks = 64; // row chunks of the parameter gradients, of a multiple of 32 rows each
 
 struct BwdRowsArgs {
   int M, nout;
@@ -24,10 +25,9 @@ struct BwdRowsArgs {
   const bf16* W2;     // [128][NO]
   const bf16* W1[2];  // [128][128] rows of W1 of the sources with a gradient
   float* dX[2];       // [M][128] their gradients
-  int mode[2];        // 0: store, 1: += what is there, 2: dX = dY' + (dX is dY)
+  int mode[2];        // 0: store, 1: += what is there, 2: dX = dY' + dH W1^T (dX may be dY)
   bf16* dH;           // [M][128]
-  bf16* dYb;          // [M][NO] BF16 of dY'
-  float* bpart;       // [blocks][kBiasCols]
+  bf16* dYb;          // [M][NO] BF16 of dY', or null
 };
 
 // One wave takes 16 rows at a time, persistent over the grid, weights in LDS
@@ -37,8 +37,8 @@ struct BwdRowsArgs {
 // channels of one row in every array it reads or writes.  The next tile's dY
 // and hidden rows are in flight over the current tile's products.
 //
-// Bound: HBM, 16 + 8 s bytes per channel and row (dY, hid, dH, dY' in BF16,
-// and 4 to 8 for each of the s dX).  The row-tiled kernel it replaces read its
+// Bound: HBM, 8 + 4 s bytes per channel and row (dY, hid, dH and the s dX; 8
+// for a dX that adds).  The row-tiled kernel it replaces read its
 // weights from L2 per wave, stored dH two bytes and dX four bytes per lane,
 // took dX of the gathered sources to HBM as FP32 (two of the three of an edge
 // MLP, 512 bytes per edge each, now k_edge_hidden_to_nodes) and left dY + add
@@ -69,11 +69,6 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void k_bwd_rows(BwdRowsArgs a) {
   const int lr = lane & 15, lg = lane >> 4, lk = 8 * lg;
   const int ntiles = (a.M + 15) / 16;
   const int stride = gridDim.x * kBwdWaves;
-  float s2[KS][8]; // this lane's column sums of dY'
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-    for (int q = 0; q < 8; ++q) s2[ks][q] = 0.f;
   struct Rows {
     float y[KS][8];
     bf16x8 h[4];
@@ -123,11 +118,8 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void k_bwd_rows(BwdRowsArgs a) {
     for (int ks = 0; ks < KS; ++ks) {
       bf16x8 yb;
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        yb[q] = (bf16)cur.y[ks][q];
-        s2[ks][q] += live ? cur.y[ks][q] : 0.f;
-      }
-      if (live && 32 * ks + lk < NO) *reinterpret_cast<bf16x8*>(a.dYb + (long)m * NO + 32 * ks + lk) = yb;
+      for (int q = 0; q < 8; ++q) yb[q] = (bf16)cur.y[ks][q];
+      if (a.dYb && live && 32 * ks + lk < NO) *reinterpret_cast<bf16x8*>(a.dYb + (long)m * NO + 32 * ks + lk) = yb;
 #pragma unroll
       for (int ub = 0; ub < 8; ++ub)
         acc[ub] = mfma(*reinterpret_cast<const bf16x8*>(&sw2[ub * 16 + lr][ks * 32 + lk]), yb, acc[ub]);
@@ -172,28 +164,6 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void k_bwd_rows(BwdRowsArgs a) {
     }
     if (tn < ntiles) cur = nxt;
   }
-  // the block's column sums: over the 16 rows of each wave, then the waves in
-  // order (the weights' LDS is free by then)
-  __syncthreads();
-  float* red = reinterpret_cast<float*>(&sw2[0][0]); // [kBwdWaves][kBiasCols], 4 KB
-  static_assert(sizeof(float) * kBwdWaves * kBiasCols <= sizeof(bf16) * kLat * (32 + 8), "the sums fit in W2's tile");
-  if (KS == 1 && lane < kLat / 2) red[w * kBiasCols + lane] = red[w * kBiasCols + kLat / 2 + lane] = 0.f;
-  if (KS == 1) wave_lds_sync();
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      float v = s2[ks][q];
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off);
-      if (lr == 0) red[w * kBiasCols + 32 * ks + lk + q] = v;
-    }
-  __syncthreads();
-  if (threadIdx.x < kBiasCols) {
-    float s = 0.f;
-    for (int k = 0; k < kBwdWaves; ++k) s += red[k * kBiasCols + threadIdx.x];
-    a.bpart[(long)blockIdx.x * kBiasCols + threadIdx.x] = s;
-  }
 }
 
 struct WgradPairArgs {
@@ -201,223 +171,368 @@ struct WgradPairArgs {
   Segs in;            // X sources of W1
   const bf16* dH;     // [M][128]
   const bf16* hid;    // [M][128]: X of W2
-  const bf16* dYb;    // [M][NO]
+  int nout;
+  const float* dY;    // dY' = dY + add[idx], as k_bwd_rows forms it
+  const float* add;
+  const int* idx;
   float* part;        // [chunks][K 128 + 128 + 128 NO]: W1, b1, W2
+  float* bpart;       // [chunks][kBiasCols]: b2
+  int y0;             // the launch's first row of blocks: 0 for W2, 1 + q for source q of W1
 };
 
-__device__ inline unsigned dword_of(const uint4& v, int d) {
-  return d == 0 ? v.x : (d == 1 ? v.y : (d == 2 ? v.z : v.w));
+// The parameter gradients are sums over all rows, added in one fixed order,
+// that of gnn_weight_grad over 64 chunks: a chunk's rows go through the MFMA
+// units 32 at a time into one accumulator, its column sums through 16 (or, for
+// up to 16 outputs, 32) interleaved chains of FP32 adds, and the chunks are
+// added in order.  Results are equal to gnn_weight_grad's bit for bit.  (An
+// order of its own, for instance rows split over a block's waves, is as exact
+// but differs in the last bits, and Adam's first steps turn a gradient that is
+// all rounding into a step of full length.)
+
+template <int C>
+struct Cols { // C consecutive BF16 columns of a row
+  unsigned d[C / 2];
+};
+template <int C>
+__device__ inline Cols<C> load_cols(const bf16* p) {
+  Cols<C> v;
+  if constexpr (C == 8) {
+    const uint4 u = *reinterpret_cast<const uint4*>(p);
+    v.d[0] = u.x;
+    v.d[1] = u.y;
+    v.d[2] = u.z;
+    v.d[3] = u.w;
+  } else if constexpr (C == 4) {
+    const uint2 u = *reinterpret_cast<const uint2*>(p);
+    v.d[0] = u.x;
+    v.d[1] = u.y;
+  } else {
+    v.d[0] = *reinterpret_cast<const unsigned*>(p);
+  }
+  return v;
 }
 
-// Column f of a lane's block of 8 rows (one row of 8, or 2, BF16 columns per
-// register group) as an MFMA fragment over the rows: one v_perm per two values.
-__device__ inline bf16x8 column_fragment(const uint4 (&r)[8], int f) {
-  uint4 o;
+// Column f of a lane's 8 rows as an MFMA fragment over the rows: one v_perm
+// per two values.
+template <int C>
+__device__ inline bf16x8 column_fragment(const Cols<C> (&r)[8], int f) {
   const unsigned sel = f & 1 ? 0x07060302u : 0x05040100u;
-  o.x = __builtin_amdgcn_perm(dword_of(r[1], f >> 1), dword_of(r[0], f >> 1), sel);
-  o.y = __builtin_amdgcn_perm(dword_of(r[3], f >> 1), dword_of(r[2], f >> 1), sel);
-  o.z = __builtin_amdgcn_perm(dword_of(r[5], f >> 1), dword_of(r[4], f >> 1), sel);
-  o.w = __builtin_amdgcn_perm(dword_of(r[7], f >> 1), dword_of(r[6], f >> 1), sel);
+  uint4 o;
+  o.x = __builtin_amdgcn_perm(r[1].d[f >> 1], r[0].d[f >> 1], sel);
+  o.y = __builtin_amdgcn_perm(r[3].d[f >> 1], r[2].d[f >> 1], sel);
+  o.z = __builtin_amdgcn_perm(r[5].d[f >> 1], r[4].d[f >> 1], sel);
+  o.w = __builtin_amdgcn_perm(r[7].d[f >> 1], r[6].d[f >> 1], sel);
   return __builtin_bit_cast(bf16x8, o);
 }
-__device__ inline bf16x8 column_fragment(const unsigned (&r)[8], int f) {
-  uint4 o;
-  const unsigned sel = f & 1 ? 0x07060302u : 0x05040100u;
-  o.x = __builtin_amdgcn_perm(r[1], r[0], sel);
-  o.y = __builtin_amdgcn_perm(r[3], r[2], sel);
-  o.z = __builtin_amdgcn_perm(r[5], r[4], sel);
-  o.w = __builtin_amdgcn_perm(r[7], r[6], sel);
-  return __builtin_bit_cast(bf16x8, o);
+
+// Row numbers m0 + 8 lg .. + 7 through idx (clamped to the chunk's last row):
+// two loads where the step is whole, of any alignment of idx.
+typedef int int4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load_rows(const int* idx, int m0, int lg, int m_end, int (&row)[8]) {
+  const int mb = m0 + 8 * lg;
+  if (m0 + 32 <= m_end) {
+    const int4u u = *reinterpret_cast<const int4u*>(idx + mb), v = *reinterpret_cast<const int4u*>(idx + mb + 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      row[j] = u[j];
+      row[4 + j] = v[j];
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) row[j] = idx[min(mb + j, m_end - 1)];
+  }
 }
 
-constexpr int kWgWaves = 4; // one per SIMD: the 128 x 128 accumulators take 256 registers a wave
+constexpr int kWgWaves = 4;
 
-// Partial dW[k][n] = sum over the block's rows of X[m][k] G[m][n], for 16 CX
-// columns of X and 16 CG of G (CX, CG columns per lane).  A wave walks 32 rows
-// at a time; lane (lr, lg) loads rows 8 lg .. + 7 at its columns CX lr .. and
-// CG lr .., whole rows being read by 16 neighbouring lanes, and turns them
-// into fragments over the rows in registers (column_fragment), so nothing is
-// transposed through LDS.  Fragment f of X holds column CX lr + f, so D row
-// 4 lg + r of product (f, g) is column CX (4 lg + r) + f of X and its column lr
-// is column CG lr + g of G.  The next rows load during the products.  The four
-// waves' sums are added in wave order through LDS at the end.
+// A wave's walk over the rows of a chunk, 32 at a time, D steps in flight.
+// load(m0, slot) loads a step's rows (clamped to the chunk's last), use(m0,
+// slot, tail) takes them; tail: some lie past the chunk's end.  The whole steps
+// run D at a time without a branch between them, so that the wait for a step
+// leaves the later ones in flight.
+template <int D, class Slot, class Load, class Use>
+__device__ __forceinline__ void walk_rows(int m_begin, int m_end, Slot (&buf)[D], Load load, Use use) {
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(m_begin + 32 * d, buf[d]);
+  int m0 = m_begin;
+  for (; m0 + 32 * D <= m_end; m0 += 32 * D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      use(m0 + 32 * d, buf[d], false);
+      load(m0 + 32 * (d + D), buf[d]);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (m0 + 32 * d < m_end) use(m0 + 32 * d, buf[d], m0 + 32 * (d + 1) > m_end);
+}
+
+template <int CX, int CG>
+__device__ __forceinline__ void store_product(const f32x4 (&acc)[CX][CG], float* out, int ldo, int lr, int lg) {
+#pragma unroll
+  for (int f = 0; f < CX; ++f)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float* p = out + (long)(CX * (4 * lg + r) + f) * ldo + CG * lr;
+      if constexpr (CG == 4)
+        *reinterpret_cast<float4*>(p) = make_float4(acc[f][0][r], acc[f][1][r], acc[f][2][r], acc[f][3][r]);
+      else if constexpr (CG == 2) *reinterpret_cast<float2*>(p) = make_float2(acc[f][0][r], acc[f][1][r]);
+      else *p = acc[f][0][r];
+    }
+}
+
+// Column sums from the chains: 0..7 of lane group 0, then of the next groups.
+template <int CG, int GROUPS>
+__device__ __forceinline__ void store_sums(const float (&cs)[8][CG], float* sum, int lr, int lg) {
+#pragma unroll
+  for (int g = 0; g < CG; ++g) {
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < GROUPS; ++k) {
+      if (k) s = __shfl(s, 16 * (k - 1) + lr);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += cs[j][g];
+    }
+    if (lg == GROUPS - 1) sum[CG * lr + g] = s;
+  }
+}
+
+// One wave of W1: dW[x0 ..][g0 ..], 16 CX columns of X by 16 CG of G = dH.  Lane
+// (lr, lg) loads rows 8 lg .. + 7 at its columns CX lr .. and CG lr .. (a row's
+// columns are read by 16 neighbouring lanes) and turns them into fragments over
+// the rows in registers (column_fragment), so nothing is transposed through
+// LDS.  Fragment f of X holds column CX lr + f, so D row 4 lg + r of product
+// (f, g) is column CX (4 lg + r) + f of X and its column lr is column CG lr + g
+// of G.  sum: the column sums of G too (db1).  A chain takes a step's rows r
+// and r + 16, which are in lanes 32 apart; the lanes lg < 2 keep the chains.
 //
-// SUM: the column sums of G too (db), each lane its rows' in FP32.
-//
-// Bound: HBM (X, G once per 128 columns of X: 512 bytes a row) beside 64 MFMAs
-// per 32 rows.
-template <int CX, int CG, bool SUM>
-__device__ __forceinline__ void wgrad_block(const bf16* X, const int* idx, int sx, const bf16* G, int sg, int m_begin,
-                                   int m_end, float* out, int ldo, float* sum, f32x4* lds) {
-  using XT = typename std::conditional<CX == 8, uint4, unsigned>::type;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+// Waves split a block's columns, not its rows (the sums' order, above), and
+// share rows through the CU's L1.  Bound: HBM beside 16 MFMAs per wave and
+// step.  Four steps in flight (32 KB a wave of 64 x 64; 18 loads a step, and a
+// wave can wait on 63).
+template <bool IDX, int CX, int CG>
+__device__ __forceinline__ void wgrad1_wave(const bf16* X, const int* idx, int sx, const bf16* G, int m_begin,
+                                            int m_end, float* out, float* sum) {
+  constexpr int D = 4;
+  const int lane = threadIdx.x & 63;
   const int lr = lane & 15, lg = lane >> 4;
   f32x4 acc[CX][CG];
 #pragma unroll
   for (int f = 0; f < CX; ++f)
 #pragma unroll
     for (int g = 0; g < CG; ++g) acc[f][g] = f32x4{0.f, 0.f, 0.f, 0.f};
-  static_assert(!SUM || CG == 8, "column sums of 128 columns only");
-  float cs[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  struct Raw {
-    XT x[8];
-    uint4 g8[CG == 8 ? 8 : 1];
-    bf16 g1[CG == 8 ? 1 : 8];
-  };
-  auto load = [&](int m0, Raw& R) {
-    const int mb = m0 + 8 * lg;
+  float cs[8][CG];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+#pragma unroll
+    for (int g = 0; g < CG; ++g) cs[j][g] = 0.f;
+  struct Slot {
+    Cols<CX> x[8];
+    Cols<CG> g[8];
+    int row[8]; // X's rows of the step that loads next into this slot
+  } buf[D];
+  if constexpr (IDX) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load_rows(idx, m_begin + 32 * d, lg, m_end, buf[d].row);
+  }
+  auto load = [&](int m0, Slot& R) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int m = mb + j < m_end ? mb + j : m_end - 1;
-      const long row = idx ? idx[m] : m;
-      R.x[j] = *reinterpret_cast<const XT*>(X + row * sx + CX * lr);
-      if constexpr (CG == 8) R.g8[j] = *reinterpret_cast<const uint4*>(G + (long)m * sg + 8 * lr);
-      else R.g1[j] = G[(long)m * sg + lr];
+      const int m = min(m0 + 8 * lg + j, m_end - 1);
+      R.x[j] = load_cols<CX>(X + (long)(IDX ? R.row[j] : m) * sx + CX * lr);
+      R.g[j] = load_cols<CG>(G + (long)m * kLat + CG * lr);
     }
-    if (m0 + 32 > m_end) { // rows past the end count nothing
+    if constexpr (IDX) load_rows(idx, m0 + 32 * D, lg, m_end, R.row);
+  };
+  auto use = [&](int m0, Slot& R, bool tail) {
+    if (tail) { // rows past the end count nothing
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        if (mb + j >= m_end) {
-          R.x[j] = XT{};
-          if constexpr (CG == 8) R.g8[j] = uint4{};
-          else R.g1[j] = (bf16)0.f;
+        if (m0 + 8 * lg + j >= m_end) {
+          R.x[j] = Cols<CX>{};
+          R.g[j] = Cols<CG>{};
         }
     }
-  };
-  int m0 = m_begin + 32 * w;
-  Raw cur, nxt;
-  if (m0 < m_end) load(m0, cur);
-  for (; m0 < m_end; m0 += 32 * kWgWaves) {
-    const int mn = m0 + 32 * kWgWaves;
-    if (mn < m_end) load(mn, nxt);
     bf16x8 gf[CG];
-    if constexpr (CG == 8) {
 #pragma unroll
-      for (int g = 0; g < CG; ++g) gf[g] = column_fragment(cur.g8, g);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) gf[0][j] = cur.g1[j];
-    }
+    for (int g = 0; g < CG; ++g) gf[g] = column_fragment<CG>(R.g, g);
 #pragma unroll
     for (int f = 0; f < CX; ++f) {
-      const bf16x8 xf = column_fragment(cur.x, f);
+      const bf16x8 xf = column_fragment<CX>(R.x, f);
 #pragma unroll
       for (int g = 0; g < CG; ++g) acc[f][g] = mfma(xf, gf[g], acc[f][g]);
     }
-    if constexpr (SUM) {
+    if (sum) {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int g = 0; g < 8; ++g) {
-          const unsigned d = dword_of(cur.g8[j], g >> 1);
-          cs[g] += __uint_as_float(g & 1 ? d & 0xffff0000u : d << 16);
+        for (int k = 0; k < CG / 2; ++k) {
+          const unsigned u = R.g[j].d[k], v = __shfl_xor(u, 32);
+          cs[j][2 * k] += __uint_as_float(u << 16);
+          cs[j][2 * k] += __uint_as_float(v << 16);
+          cs[j][2 * k + 1] += __uint_as_float(u & 0xffff0000u);
+          cs[j][2 * k + 1] += __uint_as_float(v & 0xffff0000u);
         }
-    }
-    if (mn < m_end) cur = nxt;
-  }
-  // the waves' sums, wave order, in rounds of up to four f (one per wave)
-  constexpr int FR = CX < kWgWaves ? CX : kWgWaves;
-  auto round = [&](auto first) {
-    constexpr int f0 = decltype(first)::value;
-    __syncthreads();
-#pragma unroll
-    for (int f = 0; f < FR; ++f)
-#pragma unroll
-      for (int g = 0; g < CG; ++g) lds[((w * FR + f) * CG + g) * 64 + lane] = acc[f0 + f][g];
-    __syncthreads();
-    if (w < FR) {
-      const int f = f0 + w;
-      float o[4][CG];
-#pragma unroll
-      for (int g = 0; g < CG; ++g) {
-        f32x4 s = lds[((0 * FR + w) * CG + g) * 64 + lane];
-#pragma unroll
-        for (int k = 1; k < kWgWaves; ++k) s += lds[((k * FR + w) * CG + g) * 64 + lane];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r][g] = s[r];
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float* p = out + (long)(CX * (4 * lg + r) + f) * ldo + CG * lr;
-        if constexpr (CG == 8) {
-          *reinterpret_cast<float4*>(p) = make_float4(o[r][0], o[r][1], o[r][2], o[r][3]);
-          *reinterpret_cast<float4*>(p + 4) = make_float4(o[r][4], o[r][5], o[r][6], o[r][7]);
-        } else {
-          *p = o[r][0];
-        }
-      }
     }
   };
-  round(std::integral_constant<int, 0>{});
-  if constexpr (CX > FR) round(std::integral_constant<int, FR>{});
-  if constexpr (SUM) {
-    float* ls = reinterpret_cast<float*>(lds); // [4 waves x 4 row groups][128]
-    __syncthreads();
-#pragma unroll
-    for (int g = 0; g < 8; ++g) ls[(w * 4 + lg) * kLat + 8 * lr + g] = cs[g];
-    __syncthreads();
-    if (threadIdx.x < kLat) {
-      float s = ls[threadIdx.x];
-      for (int k = 1; k < 4 * kWgWaves; ++k) s += ls[k * kLat + threadIdx.x];
-      sum[threadIdx.x] = s;
-    }
-  }
+  walk_rows<D>(m_begin, m_end, buf, load, use);
+  store_product<CX, CG>(acc, out, kLat, lr, lg);
+  if (sum) store_sums<CG, 2>(cs, sum, lr, lg);
 }
 
-// Grid (chunks, 128-wide blocks of X + 1): the last row of blocks is W2.
-// CX1: columns of X per lane for W1 (8: sources of 128, 2: one of 32);
-// CG2: columns of dY' per lane (8: 128 outputs, 1: 16).
-template <int CX1, int CG2>
+// One wave of W2: X = hid, G = dY' in FP32 (the products take it rounded to
+// BF16, the column sums, db2, as it is).  128 outputs: a wave takes all of hid's
+// columns by 32 of dY', so that dY' is read once; two steps in flight (32 KB).
+// Up to 16 outputs (NARROW): 32 columns of hid by all of dY'; a step's 32 rows
+// are 32 chains there.
+template <bool NARROW, bool Y, bool ADD>
+__device__ __forceinline__ void wgrad2_wave(const bf16* hid, const float* dY, const float* add, const int* idx,
+                                            int nout, int m_begin, int m_end, float* out, float* sum) {
+  constexpr int CX = NARROW ? 2 : 8, CG = NARROW ? 1 : 2, D = NARROW ? 3 : 2;
+  const int lane = threadIdx.x & 63;
+  const int lr = lane & 15, lg = lane >> 4;
+  f32x4 acc[CX][CG];
+#pragma unroll
+  for (int f = 0; f < CX; ++f)
+#pragma unroll
+    for (int g = 0; g < CG; ++g) acc[f][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float cs[8][CG];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+#pragma unroll
+    for (int g = 0; g < CG; ++g) cs[j][g] = 0.f;
+  typedef float V __attribute__((ext_vector_type(CG)));
+  struct Slot {
+    Cols<CX> x[8];
+    V y[8], z[8];
+    int row[8]; // add's rows of the step that loads next into this slot
+  } buf[D];
+  if constexpr (ADD) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load_rows(idx, m_begin + 32 * d, lg, m_end, buf[d].row);
+  }
+  auto load = [&](int m0, Slot& R) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int m = min(m0 + 8 * lg + j, m_end - 1);
+      R.x[j] = load_cols<CX>(hid + (long)m * kLat + CX * lr);
+      if constexpr (NARROW) R.y[j] = V(dY[(long)m * nout + min(lr, nout - 1)]);
+      else if constexpr (Y) R.y[j] = *reinterpret_cast<const V*>(dY + (long)m * kLat + CG * lr);
+      if constexpr (ADD) R.z[j] = *reinterpret_cast<const V*>(add + (long)R.row[j] * kLat + CG * lr);
+    }
+    if constexpr (ADD) load_rows(idx, m0 + 32 * D, lg, m_end, R.row);
+  };
+  auto use = [&](int m0, Slot& R, bool tail) {
+    V y[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      y[j] = V(0.f);
+      if constexpr (NARROW) {
+        if (lr < nout) y[j] = R.y[j];
+      } else if constexpr (Y) {
+        y[j] = R.y[j];
+      }
+      if constexpr (ADD) y[j] += R.z[j];
+    }
+    if (tail) { // rows past the end count nothing
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (m0 + 8 * lg + j >= m_end) {
+          R.x[j] = Cols<CX>{};
+          y[j] = V(0.f);
+        }
+    }
+    bf16x8 gf[CG];
+#pragma unroll
+    for (int g = 0; g < CG; ++g)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) gf[g][j] = (bf16)y[j][g];
+#pragma unroll
+    for (int f = 0; f < CX; ++f) {
+      const bf16x8 xf = column_fragment<CX>(R.x, f);
+#pragma unroll
+      for (int g = 0; g < CG; ++g) acc[f][g] = mfma(xf, gf[g], acc[f][g]);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int g = 0; g < CG; ++g) {
+        cs[j][g] += y[j][g];
+        if constexpr (!NARROW) cs[j][g] += __shfl_xor(y[j][g], 32);
+      }
+  };
+  walk_rows<D>(m_begin, m_end, buf, load, use);
+  store_product<CX, CG>(acc, out, NARROW ? 16 : kLat, lr, lg);
+  if (sum) store_sums<CG, NARROW ? 4 : 2>(cs, sum, lr, lg);
+}
+
+// What dY' is made of.
+enum { kDyNarrow, kDyOnly, kAddOnly, kDyAndAdd };
+
+// Grid (chunks padded to a multiple of 8, 128-wide blocks of W2 and X).  The
+// blocks of a chunk read the same rows of dH, and with eight XCDs taking blocks
+// in turn they share one's L2.  X128: sources of 128 columns (else one of 32).
+//
+// Measured: the edge MLP 38 us at 54,000 edges (44 with the rows split over the
+// waves, one step in flight and the waves' sums added through 128 KB of LDS) and
+// the node MLP 11 us at 9,240 nodes (19).  At 374,000 edges 250 us either way,
+// but W2 now reads dY' itself, so that k_bwd_rows need not write it in BF16 (155
+// -> 128 us) nor sum its columns.
+template <bool X128, int DY>
 __global__ __launch_bounds__(64 * kWgWaves, 1) void k_wgrad_pair(WgradPairArgs a) {
-  __shared__ f32x4 lds[kWgWaves * kWgWaves * 8 * 64]; // 128 KB
   const int m_begin = blockIdx.x * a.chunk;
   const int m_end = min(a.M, m_begin + a.chunk);
+  if (m_begin >= m_end) return;
   float* part = a.part + (long)blockIdx.x * ((long)(a.K + 1) * kLat + (long)kLat * a.NO);
   float* b1 = part + (long)a.K * kLat;
-  if (blockIdx.y + 1 == gridDim.y) {
-    wgrad_block<8, CG2, false>(a.hid, nullptr, kLat, a.dYb, a.NO, m_begin, m_end, b1 + kLat, a.NO, nullptr, lds);
-  } else if (blockIdx.y == 0) {
-    wgrad_block<CX1, 8, true>(a.in.src[0], a.in.idx[0], a.in.width[0], a.dH, kLat, m_begin, m_end, part, kLat, b1,
-                              lds);
+  float* b2 = a.bpart + (long)blockIdx.x * kBiasCols;
+  const int w = threadIdx.x >> 6;
+  const int c32 = 32 * w;
+  if (blockIdx.y + a.y0 == 0) {
+    float* w2 = b1 + kLat;
+    if constexpr (DY == kDyNarrow)
+      wgrad2_wave<true, true, false>(a.hid + c32, a.dY, nullptr, nullptr, a.nout, m_begin, m_end, w2 + c32 * 16,
+                                     w == 0 ? b2 : nullptr);
+    else
+      wgrad2_wave<false, DY != kAddOnly, DY != kDyOnly>(a.hid, a.dY + c32, a.add + c32, a.idx, kLat, m_begin, m_end,
+                                                        w2 + c32, b2 + c32);
+    return;
+  }
+  const int q = blockIdx.y + a.y0 - 1;
+  float* out = part + (long)a.in.start[q] * kLat;
+  if constexpr (X128) {
+    const int x64 = 64 * (w >> 1), g64 = 64 * (w & 1);
+    const bf16* X = a.in.src[q] + x64;
+    float* o = out + x64 * kLat + g64;
+    float* sum = q == 0 && x64 == 0 ? b1 + g64 : nullptr;
+    if (a.in.idx[q]) wgrad1_wave<true, 4, 4>(X, a.in.idx[q], kLat, a.dH + g64, m_begin, m_end, o, sum);
+    else wgrad1_wave<false, 4, 4>(X, nullptr, kLat, a.dH + g64, m_begin, m_end, o, sum);
   } else {
-    const int q = blockIdx.y;
-    wgrad_block<CX1, 8, false>(a.in.src[q], a.in.idx[q], a.in.width[q], a.dH, kLat, m_begin, m_end,
-                               part + (long)a.in.start[q] * kLat, kLat, nullptr, lds);
+    if (a.in.idx[0])
+      wgrad1_wave<true, 2, 2>(a.in.src[0], a.in.idx[0], 32, a.dH + c32, m_begin, m_end, out + c32, b1 + c32);
+    else wgrad1_wave<false, 2, 2>(a.in.src[0], nullptr, 32, a.dH + c32, m_begin, m_end, out + c32, b1 + c32);
   }
 }
 
-// grad (W1 | b1 | W2 | b2) = the partials summed in chunk order.  A block
-// takes 128 consecutive columns of one vector: 32 lanes of four columns by 8
-// groups of consecutive chunks, the groups added in order at the end, so that
-// eight chunks load at a time where one thread per column chained them all.
-__global__ __launch_bounds__(kThreads) void k_grad_reduce(const float* part, int nch, const float* bpart, int nb,
-                                                          int K, int NO, float* grad) {
-  __shared__ float4 red[8][32];
-  const int c = threadIdx.x & 31, g = threadIdx.x >> 5;
+// grad (W1 | b1 | W2 | b2) = the partials summed in chunk order: one column a
+// thread, 32 chunks loading at a time.
+__global__ __launch_bounds__(kThreads) void k_grad_reduce(const float* part, int nch, const float* bpart, int K,
+                                                          int NO, float* grad) {
   const long cw = (long)(K + 1) * kLat + (long)kLat * NO;
-  const long b = blockIdx.x * (long)kLat; // first column; b2 follows the others
-  const bool b2 = b >= cw;
-  const float* src = b2 ? bpart : part + b;
-  const long stride = b2 ? kBiasCols : cw;
-  const int count = b2 ? nb : nch, cols = b2 ? NO : kLat;
-  const int per = (count + 7) / 8;
-  const int k0 = g * per, k1 = min(count, k0 + per);
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 8
-  for (int k = k0; k < k1; ++k) {
-    const float4 v = *reinterpret_cast<const float4*>(src + k * stride + 4 * c);
-    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-  }
-  red[g][c] = s;
-  __syncthreads();
-  if (g == 0 && 4 * c < cols) {
+  const long c = (long)blockIdx.x * kThreads + threadIdx.x;
+  if (c >= cw + NO) return;
+  const float* src = c < cw ? part + c : bpart + (c - cw); // b2 follows the others
+  const long stride = c < cw ? cw : kBiasCols;
+  float s = 0.f;
+  for (int k0 = 0; k0 < nch; k0 += 32) {
+    float v[32];
 #pragma unroll
-    for (int k = 1; k < 8; ++k) {
-      const float4 v = red[k][c];
-      s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-    }
-    *reinterpret_cast<float4*>(grad + b + 4 * c) = s;
+    for (int k = 0; k < 32; ++k) v[k] = src[min(k0 + k, nch - 1) * stride];
+#pragma unroll
+    for (int k = 0; k < 32; ++k)
+      if (k0 + k < nch) s += v[k];
   }
+  grad[c] = s;
 }
 
 struct EdgeToNodesArgs {

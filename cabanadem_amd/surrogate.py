@@ -374,10 +374,9 @@ class Network:
             self.hid_enc_n = z(N, LAT) if train else None
             self.hid_dec = z(N, LAT) if train else None
             if train:
-                self.d_h = z(N, LAT, dt=f32)
+                self.d_h = [z(N, LAT, dt=f32) for _ in range(2)]
                 self.d_agg = z(N, LAT, dt=f32)
                 self.dH_n = z(N, LAT)
-                self.dY_n = z(N, LAT)
         if grow_e or first_train:
             E = max(E * 5 // 4, self.cap_E) if grow_e else self.cap_E
             self.cap_E = E
@@ -385,9 +384,8 @@ class Network:
             self.hid_e = [z(E, LAT) for _ in range(L)] if train else [None] * L
             self.hid_enc_e = z(E, LAT) if train else None
             if train:
-                self.d_e = z(E, LAT, dt=f32)
+                self.d_e = [z(E, LAT, dt=f32) for _ in range(2)]
                 self.dH_e = z(E, LAT)
-                self.dY_e = z(E, LAT)
         if train and self.work is None:
             self.work = torch.empty(GRAD_WORK_FLOATS, dtype=f32, device=dev)
 
@@ -470,40 +468,44 @@ class Network:
         Lb, s, N, E = glib(), stream(), g.N, g.E
         F = self.flat
         base = self.grad.data_ptr()
-        d_h, d_agg, d_e = self.d_h, self.d_agg, self.d_e
+        # a gradient that an MLP adds to goes from one of two buffers to the
+        # other, so that W2's gradient can read dY beside W1's
+        (d_h, h2), (d_e, e2), d_agg = self.d_h, self.d_e, self.d_agg
 
-        def grads(mlp, inp, dY, add, idx, hid, dX, acc, dH, dYb):
+        def grads(mlp, inp, dY, add, idx, hid, dX, acc, dH):
             _ok(Lb.gnn_mlp_grads(C.byref(inp), C.byref(mlp.weights(F)), ptr(dY), ptr(add), ptr(idx), ptr(hid),
                                  (C.c_void_p * 3)(*[None if d is None else d.data_ptr() for d in dX]), acc,
-                                 ptr(dH), ptr(dYb), ptr(self.work), GRAD_WORK_FLOATS,
+                                 ptr(dH), None, ptr(self.work), GRAD_WORK_FLOATS,
                                  C.c_void_p(base + 4 * mlp.o_W1), s), "mlp gradients")
 
         none3 = (None, None, None)
+        residual = 8  # dX of the first source = dY + ...
         grads(self.dec, io(N, (self.h[self.L], None)), d_out, None, None, self.hid_dec, (d_h, None, None), 0,
-              self.dH_n, self.dY_n)
+              self.dH_n)
         for l in reversed(range(self.L)):
             h, e = self.h[l], self.e[l]
-            # node MLP: h_{l+1} = h_l + MLP_n([h_l, agg_l]); the residual
-            # source adds into d_h (accumulate bit 0), d_agg is overwritten
+            # node MLP: h_{l+1} = h_l + MLP_n([h_l, agg_l])
             grads(self.node[l], io(N, (h, None), (self.agg[l], None)), d_h, None, None, self.hid_n[l],
-                  (d_h, d_agg, None), 1, self.dH_n, self.dY_n)
+                  (h2, d_agg, None), residual, self.dH_n)
+            d_h, h2 = h2, d_h
             if E > 0:
                 # edge MLP: e_{l+1} = e_l + MLP_e([e_l, h_l[recv], h_l[send]]),
                 # aggregated into agg_l: d_e(l+1) += d_agg[recv] on the way in
                 # (nothing but that for the last layer)
                 grads(self.edge[l], io(E, (e, None), (h, g.recv), (h, g.send)), d_e if l + 1 < self.L else None,
-                      d_agg, g.recv, self.hid_e[l], (d_e, None, None), 1, self.dH_e, self.dY_e)
+                      d_agg, g.recv, self.hid_e[l], (e2, None, None), residual, self.dH_e)
+                d_e, e2 = e2, d_e
                 _ok(Lb.gnn_edge_hidden_grad_to_nodes(N, ptr(self.dH_e), ptr(g.row), ptr(g.rev),
                                                      C.byref(self.edge[l].weights(F)), ptr(d_h), s),
                     "edge grads to nodes")
         # encoders (their inputs are data: no input gradient)
         if E > 0:
-            grads(self.enc_e, io(E, (xe, None)), d_e, None, None, self.hid_enc_e, none3, 0, self.dH_e, self.dY_e)
+            grads(self.enc_e, io(E, (xe, None)), d_e, None, None, self.hid_enc_e, none3, 0, self.dH_e)
         else:
             self._zero_grad(self.enc_e)
             for l in range(self.L):
                 self._zero_grad(self.edge[l])
-        grads(self.enc_n, io(N, (xn, None)), d_h, None, None, self.hid_enc_n, none3, 0, self.dH_n, self.dY_n)
+        grads(self.enc_n, io(N, (xn, None)), d_h, None, None, self.hid_enc_n, none3, 0, self.dH_n)
 
     def _zero_grad(self, mlp):
         self.grad[mlp.o_W1:mlp.end].zero_()

@@ -76,20 +76,20 @@ int gnn_mlp_backward(const gnn_mlp_io* io, const gnn_mlp_weights* w, const float
 int gnn_weight_grad(const gnn_mlp_io* io, const void* G_bf16, const float* G_f32, int ncols,
                     int ncols_pad, float* part, float* bpart, int nchunks, float* dW, float* db,
                     int accumulate, void* stream);
-/* The whole backward of one MLP of the network, parameter gradients included
- * (up to the FP32 order of those sums the same as gnn_broadcast_add,
- * gnn_mlp_backward and two gnn_weight_grad):
+/* The whole backward of one MLP of the network, parameter gradients included:
+ * bit for bit gnn_broadcast_add, gnn_mlp_backward and two gnn_weight_grad over
+ * 64 chunks.
  *   dY' = dY + add[add_idx]  (add: float [.][128], NULL: none; dY NULL: zero),
- *   dH = (dY' W2^T) masked by hidden > 0, bf16 [M][128];  dYb = dY' as bf16
- *   [M][nout_pad] (both outputs: work arrays of the caller's),
+ *   dH = (dY' W2^T) masked by hidden > 0, bf16 [M][128] (output, a work array
+ *   of the caller's);  dYb = dY' as bf16 [M][nout_pad], NULL to skip,
  *   dX[q] (float [M][128], NULL to skip, two at most) = dH W1^T restricted to
- *   source q, stored, or added when bit q of accumulate is set; a source whose
- *   dX is dY (or dY NULL) gets dY' + dH W1^T, as a residual does,
+ *   source q, stored, or added when bit q of accumulate is set (where dX[q] is
+ *   dY, or dY NULL, to dY'); bit 3 + q (128 outputs): dX[q] = dY' + dH W1^T, as
+ *   a residual needs it.  dX[q] = dY costs a launch more; add is none of the dX,
  *   grad = W1 [K][128] | b1 [128] | W2 [128][nout_pad] | b2 [nout_pad].
  * Sources: each 128 wide (gathered or not), or one of 32 without dX; 128
  * outputs, or up to 16 (nout_pad 16, no add).  Arrays 16-byte aligned.
- * work: GNN_GRAD_WORK_FLOATS floats cover every shape on a GPU of up to 256
- * compute units.  Deterministic. */
+ * work: GNN_GRAD_WORK_FLOATS floats cover every shape.  Deterministic. */
 #define GNN_GRAD_WORK_FLOATS (5L * 1024L * 1024L)
 int gnn_mlp_grads(const gnn_mlp_io* io, const gnn_mlp_weights* w, const float* dY, const float* add,
                   const int* add_idx, const void* hidden, float* const dX[3], int accumulate, void* dH,
