@@ -18,6 +18,7 @@ constexpr int kGradChunks = 64; // row chunks of the parameter gradients, of a m
 
 struct BwdRowsArgs {
   int M, nout;
+  int per;            // tiles a block takes side by side (one per wave, at most its waves)
   const float* dY;    // [M][nout], or null (zeros, with add)
   const float* add;   // [.][128] rows added through idx, or null
   const int* idx;     // [M]
@@ -68,17 +69,24 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void k_bwd_rows(BwdRowsArgs a) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int lr = lane & 15, lg = lane >> 4, lk = 8 * lg;
   const int ntiles = (a.M + 15) / 16;
-  const int stride = gridDim.x * kBwdWaves;
+  const int stride = gridDim.x * a.per;
   struct Rows {
     float y[KS][8];
     bf16x8 h[4];
+  };
+  // add's row of the tile that loads next: loads are waited for in the order of
+  // their issue and stand outside branches (the last tile has a copy of the code
+  // without them), so that a tile does not wait for the next one's rows
+  int ai = 0;
+  auto load_index = [&](int t) {
+    if (a.add) ai = a.idx[t * 16 + lr < a.M ? t * 16 + lr : a.M - 1];
   };
   auto load = [&](int t, Rows& R) {
     const int m = t * 16 + lr < a.M ? t * 16 + lr : a.M - 1; // clamped loads; stores are guarded
 #pragma unroll
     for (int s4 = 0; s4 < 4; ++s4) R.h[s4] = ld8(a.hid + (long)m * kLat + 32 * s4 + lk);
     if constexpr (NO == kLat) {
-      const float* add = a.add ? a.add + (long)a.idx[m] * kLat + lk : nullptr;
+      const float* add = a.add ? a.add + (long)ai * kLat + lk : nullptr;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         float4 u = make_float4(0.f, 0.f, 0.f, 0.f), v = u;
@@ -101,12 +109,17 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void k_bwd_rows(BwdRowsArgs a) {
       for (int q = 0; q < 8; ++q) R.y[0][q] = lk + q < a.nout ? a.dY[(long)m * a.nout + lk + q] : 0.f;
     }
   };
-  int t = blockIdx.x * kBwdWaves + w;
+  int t = blockIdx.x * a.per + w;
+  if (w >= a.per || t >= ntiles) return;
   Rows cur, nxt;
-  if (t < ntiles) load(t, cur);
-  for (; t < ntiles; t += stride) {
-    const int tn = t + stride;
-    if (tn < ntiles) load(tn, nxt);
+  load_index(t);
+  load(t, cur);
+  load_index(min(t + stride, ntiles - 1));
+  auto tile = [&](int t, auto more) {
+    if constexpr (decltype(more)::value) {
+      load(t + stride, nxt);
+      load_index(min(t + 2 * stride, ntiles - 1));
+    }
     // keeps the weight fragments' LDS reads inside the loop
     __asm__ volatile("" ::: "memory");
     const int m = t * 16 + lr;
@@ -162,8 +175,12 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void k_bwd_rows(BwdRowsArgs a) {
         *reinterpret_cast<float4*>(p) = o;
       }
     }
-    if (tn < ntiles) cur = nxt;
+  };
+  for (; t + stride < ntiles; t += stride) {
+    tile(t, std::true_type{});
+    cur = nxt;
   }
+  tile(t, std::false_type{});
 }
 
 struct WgradPairArgs {
@@ -537,6 +554,7 @@ __global__ __launch_bounds__(kThreads) void k_grad_reduce(const float* part, int
 
 struct EdgeToNodesArgs {
   int N;
+  int per;            // groups of nodes a block takes side by side (one per wave, at most its waves)
   const bf16* dH;     // [E][128]
   const int* row;     // [N + 1]
   const int* rev;     // [E]
@@ -556,6 +574,9 @@ constexpr int kToNodesPitch = kLat + 4; // floats; rows 16 bytes aligned, banks 
 // channels edge by edge into the running sum of the current node.  The edges'
 // FP32 gradients (2 x 512 bytes per edge written and read back by the two
 // kernels this replaces) never leave the chip: 2 x 256 bytes per edge are read.
+// What a node needs besides (its dh row, its edges' end) and the reverse edges
+// are loaded ahead: loaded when reached, each cost its wave a round trip per
+// node (31 -> 25 us at 54,000 edges, 124 -> 98 at 374,000).
 __global__ __launch_bounds__(64 * kToNodesWaves, 1) void k_edge_hidden_to_nodes(EdgeToNodesArgs a) {
   __shared__ bf16 swb[kLat][kWPitch], swc[kLat][kWPitch]; // W1b, W1c: [row][u], rows in unit_of_row order
   __shared__ float st[kToNodesWaves][2][16][kToNodesPitch];
@@ -568,34 +589,44 @@ __global__ __launch_bounds__(64 * kToNodesWaves, 1) void k_edge_hidden_to_nodes(
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int lr = lane & 15, lg = lane >> 4, lk = 8 * lg;
   const int groups = (a.N + 15) / 16;
-  for (int grp = blockIdx.x * kToNodesWaves + w; grp < groups; grp += gridDim.x * kToNodesWaves) {
+  if (w >= a.per) return;
+  for (int grp = blockIdx.x * a.per + w; grp < groups; grp += gridDim.x * a.per) {
     // keeps the weight fragments' LDS reads inside the loop
     __asm__ volatile("" ::: "memory");
     const int n0 = grp * 16, n1 = min(a.N, n0 + 16);
-    const int e_end = __builtin_amdgcn_readfirstlane(a.row[n1]);
-    int e0 = __builtin_amdgcn_readfirstlane(a.row[n0]);
-    int n = n0, end = __builtin_amdgcn_readfirstlane(a.row[n0 + 1]);
+    const int ends = a.row[min(n0 + lane, n1)]; // lane k: the first edge of node n0 + k
+    const int e_end = __builtin_amdgcn_readlane(ends, n1 - n0);
+    int e0 = __builtin_amdgcn_readlane(ends, 0);
+    int n = n0, end = __builtin_amdgcn_readlane(ends, 1);
     float sx = 0.f, sy = 0.f;
+    // this node's and the next one's dh, loaded two nodes ahead
+    auto node_row = [&](int k) { return reinterpret_cast<float2*>(a.dh + (long)min(k, n1 - 1) * kLat + 2 * lane); };
+    float2 d0 = *node_row(n0), d1 = *node_row(n0 + 1);
     auto flush = [&]() { // node n is complete: add it and go to the next
-      float2* p = reinterpret_cast<float2*>(a.dh + (long)n * kLat + 2 * lane);
-      float2 v = *p;
-      v.x += sx; v.y += sy;
-      *p = v;
+      d0.x += sx; d0.y += sy;
+      *node_row(n) = d0;
       sx = sy = 0.f;
       ++n;
-      end = n < n1 ? __builtin_amdgcn_readfirstlane(a.row[n + 1]) : INT_MAX;
+      d0 = d1;
+      if (n + 1 < n1) d1 = *node_row(n + 1);
+      end = n < n1 ? __builtin_amdgcn_readlane(ends, n - n0 + 1) : INT_MAX;
     };
     bf16x8 Br[4], Bs[4];
+    int er = 0; // the reverse edge of the next tile's
+    auto clamped = [&](int e) { return min(e + lr, e_end - 1); };
     auto load = [&](int e) {
-      const int ee = e + lr < e_end ? e + lr : e_end - 1;
-      const int er = a.rev[ee];
+      const int ee = clamped(e);
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
         Br[ks] = ld8(a.dH + (long)ee * kLat + 32 * ks + lk);
         Bs[ks] = ld8(a.dH + (long)er * kLat + 32 * ks + lk);
       }
+      er = a.rev[clamped(e + 16)];
     };
-    if (e0 < e_end) load(e0);
+    if (e0 < e_end) {
+      er = a.rev[clamped(e0)];
+      load(e0);
+    }
     for (; e0 < e_end; e0 += 16) {
       f32x4 r[8], s[8];
 #pragma unroll
@@ -615,13 +646,18 @@ __global__ __launch_bounds__(64 * kToNodesWaves, 1) void k_edge_hidden_to_nodes(
         *reinterpret_cast<f32x4*>(&st[w][1][lr][c]) = s[ub];
       }
       wave_lds_sync();
-      const int cnt = min(16, e_end - e0);
-      for (int k = 0; k < cnt; ++k) {
+      float2 u[16], v[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        u[k] = *reinterpret_cast<const float2*>(&st[w][0][k][2 * lane]);
+        v[k] = *reinterpret_cast<const float2*>(&st[w][1][k][2 * lane]);
+      }
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        if (e0 + k >= e_end) break;
         while (e0 + k >= end) flush();
-        const float2 u = *reinterpret_cast<const float2*>(&st[w][0][k][2 * lane]);
-        const float2 v = *reinterpret_cast<const float2*>(&st[w][1][k][2 * lane]);
-        sx += u.x; sy += u.y;
-        sx += v.x; sy += v.y;
+        sx += u[k].x; sy += u[k].y;
+        sx += v[k].x; sy += v[k].y;
       }
       wave_lds_sync(); // the next tile rewrites the sums
     }
