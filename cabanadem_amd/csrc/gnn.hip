@@ -1215,6 +1215,42 @@ __global__ __launch_bounds__(kThreads) void k_cast_weights(const float* p, int K
   Wt[(long)n * K + k] = v;
 }
 
+struct CastAllArgs {
+  const float* p;    // the flat FP32 parameters
+  bf16* out;         // [K][NP] and its transpose [NP][K] of each matrix
+  const int* table;  // per matrix: first parameter, K, N, NP, first value in out
+};
+
+// k_cast_weights for all matrices in one launch (blockIdx.y), in tiles of 64 k
+// by 16 n turned over in LDS, so that both copies are written 8 bytes a lane.
+// 46 launches of k_cast_weights, each a few blocks whose lanes wrote the
+// transpose two bytes to a line, took 150 us of a ten-layer training step.
+constexpr int kCastK = 64, kCastN = 16;
+__global__ __launch_bounds__(kThreads) void k_cast_all(CastAllArgs a) {
+  __shared__ bf16 st[kCastN][kCastK + 4];
+  const int* d = a.table + 5 * blockIdx.y;
+  const int K = d[1], N = d[2], NP = d[3];
+  const int kt = (K + kCastK - 1) / kCastK, tiles = kt * (NP / kCastN);
+  if ((int)blockIdx.x >= tiles) return;
+  const int k0 = (int)blockIdx.x % kt * kCastK, n0 = (int)blockIdx.x / kt * kCastN;
+  bf16 *W = a.out + d[4], *Wt = W + (long)K * NP;
+  const int k = threadIdx.x >> 2, n4 = (threadIdx.x & 3) * 4;
+  if (k0 + k < K) {
+    const float* p = a.p + d[0] + (long)(k0 + k) * NP + n0 + n4;
+    bf16x4 v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      v[q] = (bf16)(n0 + n4 + q < N ? p[q] : 0.f);
+      st[n4 + q][k] = v[q];
+    }
+    *reinterpret_cast<bf16x4*>(W + (long)(k0 + k) * NP + n0 + n4) = v;
+  }
+  __syncthreads();
+  const int n = threadIdx.x >> 4, k4 = (threadIdx.x & 15) * 4;
+  if (k0 + k4 < K)
+    *reinterpret_cast<bf16x4*>(Wt + (long)(n0 + n) * K + k0 + k4) = *reinterpret_cast<const bf16x4*>(&st[n][k4]);
+}
+
 // Mean squared error over M x C values: dY = 2 (y - t) / (M C) and per-block
 // partial sums of (y - t)^2.
 __global__ __launch_bounds__(kThreads) void k_mse(const float* y, const float* t, long count,
@@ -1931,6 +1967,15 @@ int gnn_adam(float* p, const float* g, float* m, float* v, long n, float lr_t, f
   if (!p || !g || !m || !v || n <= 0) return -1;
   hipLaunchKernelGGL(k_adam, dim3(nblk(n)), dim3(kThreads), 0, reinterpret_cast<hipStream_t>(stream),
                      p, g, m, v, n, lr_t, b1, b2, eps, wd);
+  return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+int gnn_cast_all(const float* p, void* out, const int* table, int count, int max_elements, void* stream) {
+  if (!p || !out || !table || count <= 0 || max_elements <= 0 || (reinterpret_cast<uintptr_t>(out) & 7)) return -1;
+  // a matrix of K rows has at most K / 64 + 1 tiles in each 16 columns
+  const int tiles = max_elements / (kCastK * kCastN) + kLat / kCastN;
+  hipLaunchKernelGGL(k_cast_all, dim3(tiles, count), dim3(kThreads), 0, reinterpret_cast<hipStream_t>(stream),
+                     (CastAllArgs{p, reinterpret_cast<bf16*>(out), table}));
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

@@ -73,6 +73,7 @@ _SIG = {
     "gnn_adam": (C.c_int, [_vp, _vp, _vp, _vp, C.c_long, C.c_float, C.c_float, C.c_float, C.c_float,
                            C.c_float, _vp]),
     "gnn_cast_weights": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, _vp, _vp, _vp]),
+    "gnn_cast_all": (C.c_int, [_vp, _vp, _vp, C.c_int, C.c_int, _vp]),
     "gnn_node_features": (C.c_int, [C.c_int, _vp, _vp, C.c_int, _vp, C.c_float, C.c_float, C.c_float,
                                     _vp, C.c_int, C.c_float, _vp, _vp]),
     "gnn_edge_features": (C.c_int, [C.c_long, _vp, _vp, _vp, C.c_double, _vp, _vp]),
@@ -234,13 +235,18 @@ class MLP:
         self.o_b2 = self.o_W2 + LAT * self.NP
         self.end = self.o_b2 + self.NP
 
-    def alloc(self, dev):
+    def alloc(self, dev, arena=None, at=0):
+        """The BF16 copies (W1, W1^T, W2, W2^T), in arena from `at` on."""
         torch = _torch()
-        bf = torch.bfloat16
-        self.W1 = torch.zeros((self.K, LAT), dtype=bf, device=dev)
-        self.W1t = torch.zeros((LAT, self.K), dtype=bf, device=dev)
-        self.W2 = torch.zeros((LAT, self.NP), dtype=bf, device=dev)
-        self.W2t = torch.zeros((self.NP, LAT), dtype=bf, device=dev)
+        if arena is None:
+            arena = torch.zeros(self.n_weights(), dtype=torch.bfloat16, device=dev)
+        self.W1, self.W1t, self.W2, self.W2t = (
+            t.view(s) for t, s in zip(arena[at:at + self.n_weights()].split(
+                [self.K * LAT] * 2 + [LAT * self.NP] * 2),
+                [(self.K, LAT), (LAT, self.K), (LAT, self.NP), (self.NP, LAT)]))
+
+    def n_weights(self):
+        return 2 * LAT * (self.K + self.NP)
 
     def views(self, flat):
         return (flat[self.o_W1:self.o_b1].view(self.K, LAT), flat[self.o_b1:self.o_W2],
@@ -315,8 +321,16 @@ class Network:
         self.m = torch.zeros_like(self.flat)
         self.v = torch.zeros_like(self.flat)
         self.t = 0
+        # the BF16 weights of all MLPs in one array, and for the cast each
+        # matrix's first parameter, K, N, NP and place in it
+        self.weights = torch.zeros(sum(m.n_weights() for m in self.mlps), dtype=torch.bfloat16, device=device)
+        table, at = [], 0
         for m in self.mlps:
-            m.alloc(device)
+            m.alloc(device, self.weights, at)
+            table += [[m.o_W1, m.K, LAT, LAT, at], [m.o_W2, LAT, m.nout, m.NP, at + 2 * m.K * LAT]]
+            at += m.n_weights()
+        self.cast_table = torch.tensor(table, dtype=torch.int32).to(device)
+        self.cast_max = max(K * NP for _, K, _, NP, _ in table)
         self.cast()
         self.cap_N = self.cap_E = 0
         self.h = self.e = None
@@ -324,13 +338,8 @@ class Network:
 
     # -- parameters --------------------------------------------------------
     def cast(self):
-        L, s = glib(), stream()
-        for m in self.mlps:
-            base = self.flat.data_ptr()
-            _ok(L.gnn_cast_weights(C.c_void_p(base + 4 * m.o_W1), m.K, LAT, LAT, ptr(m.W1), ptr(m.W1t), s),
-                "cast W1")
-            _ok(L.gnn_cast_weights(C.c_void_p(base + 4 * m.o_W2), LAT, m.nout, m.NP, ptr(m.W2), ptr(m.W2t),
-                                   s), "cast W2")
+        _ok(glib().gnn_cast_all(ptr(self.flat), ptr(self.weights), ptr(self.cast_table),
+                                self.cast_table.shape[0], self.cast_max, stream()), "cast weights")
 
     def adam(self, lr, b1=0.9, b2=0.999, eps=1e-8, wd=0.0):
         self.t += 1

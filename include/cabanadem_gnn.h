@@ -113,6 +113,12 @@ int gnn_adam(float* p, const float* g, float* m, float* v, long n, float lr_t, f
              float b2, float eps, float wd, void* stream);
 /* FP32 master [K][NP] (columns >= N are zero) -> bf16 W [K][NP] and Wt [NP][K]. */
 int gnn_cast_weights(const float* p, int K, int N, int NP, void* W, void* Wt, void* stream);
+/* gnn_cast_weights for `count` matrices of one parameter vector p in one
+ * launch.  table (device, int [count][5]): the matrix's first parameter, K, N,
+ * NP, and the place of its W (bf16 [K][NP], then Wt [NP][K]) in out; K a
+ * multiple of 4, NP of 16 and up to 128, places multiples of 4, out 8-byte
+ * aligned; max_elements: the largest K NP. */
+int gnn_cast_all(const float* p, void* out, const int* table, int count, int max_elements, void* stream);
 /* Node features (bf16 [N][32]): the H most recent velocities vhist
  * (float [H][N][3], oldest first) / v_scale, (r - r_mean) / r_scale, and
  * for each plane (float [n_planes][4] = unit normal, offset d) the distance
