@@ -898,6 +898,9 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
       stream_store<NT>(a.ch_out + (3 * m + 2) * ld + i, h[2]);
     }
   }
+  // The state staged below overwrites every lane's contact ids: all lanes of the
+  // wave have read theirs by then (the tile's contact rounds end with a barrier).
+  if (STAGE && !WAVE) wave_lds_sync();
   bool defer = false;
   if (DEFER) {
     if (act) {
