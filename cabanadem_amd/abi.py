@@ -176,6 +176,7 @@ SYMBOLS = {
     "dem_set_force_pass": (C.c_int, [C.c_void_p, C.c_int]),
     "dem_set_shape": (C.c_int, [C.c_void_p, C.c_int, C.c_int]),
     "dem_get_shape": (C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
+    "dem_get_streaming": (C.c_int, [C.c_void_p, C.POINTER(C.c_int)]),
     "dem_set_graph": (C.c_int, [C.c_void_p, C.c_int]),
     "dem_autotune": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(DemTuneResult)]),
     "dem_enable_bonds": (C.c_int, [C.c_void_p, C.POINTER(DemBondConfig)]),
@@ -501,6 +502,12 @@ class System:
         b, r = C.c_int(), C.c_int()
         self._check(self._lib.dem_get_shape(self._h, C.byref(b), C.byref(r)))
         return b.value, r.value
+
+    def streaming(self) -> bool:
+        """Whether fused steps go past the caches: dem_get_streaming."""
+        s = C.c_int()
+        self._check(self._lib.dem_get_streaming(self._h, C.byref(s)))
+        return bool(s.value)
 
     def set_params(self, **changes):
         """Non-structural dem_config fields (dt, cor_pp, ..., rebuild_every, physics_mode)."""

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(kBlock) void k_kick(StepArgs a, double4* xr, double
   }
 }
 
-__global__ __launch_bounds__(1024) void k_sample_lists(int n, const int* cmeta, const int* nbond, DevFlags* flags) {
+__global__ __launch_bounds__(1024) void k_sample_lists(int n, const int* cmeta, const int* nbond, int* out) {
   __shared__ int part[2][16];
   int c = 0, b = 0;
 #pragma unroll
@@ -135,8 +135,8 @@ __global__ __launch_bounds__(1024) void k_sample_lists(int n, const int* cmeta, 
       c += part[0][k];
       b += part[1][k];
     }
-    flags->sampled_contacts = c;
-    flags->sampled_bonds = b;
+    out[0] = c;
+    out[1] = b;
   }
 }
 
@@ -269,8 +269,8 @@ hipError_t launch_kick(const StepArgs& a, double4* xr, double* uw, const double*
   return hipGetLastError();
 }
 
-hipError_t launch_sample_lists(int n, const int* cmeta, const int* nbond, DevFlags* flags, hipStream_t s) {
-  hipLaunchKernelGGL(k_sample_lists, dim3(1), dim3(1024), 0, s, n, cmeta, nbond, flags);
+hipError_t launch_sample_lists(int n, const int* cmeta, const int* nbond, int* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_sample_lists, dim3(1), dim3(1024), 0, s, n, cmeta, nbond, out);
   return hipGetLastError();
 }
 

@@ -118,11 +118,9 @@ struct DevFlags {
   int bond_overflow;
   int cell_overflow;  // a cell held more than kMaxCellParticles particles
   int bonds_broken;   // bonds broken since the flags were last cleared
-  int sampled_contacts; // tracked contacts and bond slots of kListSamples
-  int sampled_bonds;    // particles (launch policy only)
 };
 
-// Particles whose list lengths the end of a step call samples.
+// Particles whose list lengths a sample sums (launch policy only).
 constexpr int kListSamples = 4096;
 
 // Upper bound on particles in one cell; beyond it the binning box is far too
@@ -318,9 +316,9 @@ hipError_t launch_get_kinematics(int n, const int* id, const double4* xr, const 
                                  double* u, hipStream_t s);
 hipError_t launch_kick(const StepArgs& a, double4* xr, double* uw, const double* ft,
                        int do_kick, int do_drift, hipStream_t s);
-// flags->sampled_contacts, sampled_bonds = those of kListSamples particles
-// spread over the n (nbond null: no bonds).
-hipError_t launch_sample_lists(int n, const int* cmeta, const int* nbond, DevFlags* flags, hipStream_t s);
+// out[0], out[1] = tracked contacts, bond slots (nbond null: 0) of kListSamples
+// particles spread over the n.
+hipError_t launch_sample_lists(int n, const int* cmeta, const int* nbond, int* out, hipStream_t s);
 // Per-tile partial sums of the current state (one partial row per tile).
 hipError_t launch_diag_current(const StepArgs& a, const double* uw, hipStream_t s);
 // The force kernels for one tile size each (a.block), in translation units

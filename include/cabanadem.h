@@ -357,6 +357,11 @@ int dem_set_force_pass(dem_ctx* ctx, int mode);
  * sums (results agree to rounding, as across rebuild cadences). */
 int dem_set_shape(dem_ctx* ctx, int block, int tile_rows);
 int dem_get_shape(dem_ctx* ctx, int* block, int* tile_rows);
+/* 1 while a fused step is taken to touch more than the last-level cache holds,
+ * so that its own streams go past the caches (from the particle count, the
+ * bonds, and the contacts as uploaded or last sampled).  Results do not depend
+ * on it. */
+int dem_get_streaming(dem_ctx* ctx, int* streaming);
 
 /* Captured step sequences: with enable set (and no diagnostics sampling or
  * kernel timing on), dem_step runs whole cycles of 2 rebuild_every steps
