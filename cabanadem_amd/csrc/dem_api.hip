@@ -1871,10 +1871,13 @@ int dem_autotune(dem_ctx* c, int trial_steps, dem_tune_result* out) {
   if (best > 0.) {
     const int K = out->rebuild_every, g = out->grid_blocks, graph = out->use_graph, pass = out->force_pass;
     const std::vector<int> bks = c->bonds_on ? std::vector<int>{1} : std::vector<int>{0, 1, 2};
+    // the eight-lane pass has no tiles: other blocks are tried on the one-lane
+    // kernels, which a launch grid keeps
+    const bool group = takes_group(c->n, c->bonds_on, c->n_groups > 0, pass, g);
     for (int bk : bks)
       for (int rows : {4, 8, 16})
         if (bk != snap.bidx || rows != snap.tile_rows)
-          if (int r = trial(K, g, graph, pass, bk, rows)) return r;
+          if (int r = trial(K, group && bk != snap.bidx ? grids.back() : g, graph, pass, bk, rows)) return r;
   }
   out->n_trials = nt;
   out->ms_per_step = best;

@@ -229,7 +229,8 @@ hipError_t launch_force(ForceKind kind, const StepArgs& a, bool sample, int grid
   // per step, one lane / eight: spheres in touch 1k 22 / 10, 10k 21 / 12, 33k
   // 22 / 19, 64k 30 / 27; a loose bed 10k 13.4 / 11.3, 64k 15 / 23.  The line
   // lies where neither density loses.
-  if (a.n <= kGroupMax && !bond && !sample && !a.vgroup && !a.split && !a.wave && grid_blocks == 0 &&
+  const int pass = a.split ? DEM_FORCE_PASS_SPLIT : (a.wave ? DEM_FORCE_PASS_WAVE : DEM_FORCE_PASS_FUSED);
+  if (takes_group(a.n, bond, a.vgroup != nullptr, pass, grid_blocks) && !sample &&
       (kind == FK_PP_PW_FORCES || kind == FK_STEP_FUSED || kind == FK_STEP_LAST))
     return launch_force_group(ref, kind, a, s);
   switch (a.block) {

@@ -308,6 +308,11 @@ hipError_t launch_force_group(bool ref, ForceKind kind, const StepArgs& a, hipSt
 #define DEM_GROUP_MAX 20000
 #endif
 constexpr int kGroupMax = DEM_GROUP_MAX;
+// Whether unsampled whole force passes take it: the default force pass and
+// launch (a grid keeps the kernels of one lane per particle).
+inline bool takes_group(int n, bool bonds, bool groups, int force_pass, int grid_blocks) {
+  return n <= kGroupMax && !bonds && !groups && force_pass == DEM_FORCE_PASS_FUSED && grid_blocks == 0;
+}
 hipError_t launch_zero_forces(const StepArgs& a, hipStream_t s);
 hipError_t launch_update_tangential(const StepArgs& a, hipStream_t s);
 hipError_t launch_set_kinematics(int n, const int* id, const double* x, const double* u, int clear,

@@ -348,6 +348,8 @@ int dem_set_force_pass(dem_ctx* ctx, int mode);
 
 /* Tile shapes.  block: the force kernels' workgroup size and tile of
  * consecutive slots, 64, 128 or 256 (0: 128; systems with bonds run 128).
+ * The eight-lane pass of up to 20,000 particles (dem_set_launch) has no
+ * tiles and ignores it.
  * tile_rows: the binning grid numbers its cells in y-tiles of tile_rows
  * full x-rows, z-major inside a tile (1 to 32; 0: 8), which sets how far
  * apart in memory the z-neighbours of a particle sit after the re-sort.
@@ -380,7 +382,8 @@ int dem_set_graph(dem_ctx* ctx, int enable);
  * on or off and force-pass shape (DEM_FORCE_PASS_*, systems without bonds)
  * at the context's tile shapes; stage 2 tries, at the best of stage 1, the
  * tile shapes of dem_set_shape: blocks of 64, 128 and 256 (systems without
- * bonds) times cell tiles of 4, 8 and 16 rows.  Rebuild cadence and cell
+ * bonds; where stage 1 chose the eight-lane pass, other blocks with the last
+ * of the grids) times cell tiles of 4, 8 and 16 rows.  Rebuild cadence and cell
  * tiles change the summation order of the contact sums after a re-sort, so
  * runs with different ones agree to rounding, not bitwise. */
 #define DEM_TUNE_MAX_TRIALS 128
