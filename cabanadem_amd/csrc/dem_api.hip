@@ -1093,6 +1093,7 @@ int dem_set_system_params(dem_ctx* c, int system, double cor_pp, double cor_pw,
   if (c->nsys == 1) {
     c->cfg.cor_pp = cor_pp; c->cfg.cor_pw = cor_pw;
     c->cfg.friction_pp = friction_pp; c->cfg.friction_pw = friction_pw;
+    ++c->gen; // captured launches carry one system's materials
   }
   return c->upload_sys();
 }
