@@ -1860,7 +1860,7 @@ int gnn_mlp_grads(const gnn_mlp_io* io, const gnn_mlp_weights* wt, const float* 
   const bool narrow = io->nseg == 1 && io->width[0] == 32;
   if (K != wt->K) return -1;
   for (int q = 0; q < io->nseg; ++q)
-    if ((io->width[q] != kLat && !narrow) || !aligned16(io->src[q])) return -1;
+    if (!narrow && (io->width[q] != kLat || !aligned16(io->src[q]))) return -1;
   if (!aligned16(dY) && wide) return -1;
   if (!aligned16(add) || !aligned16(hidden) || !aligned16(dH) || !aligned16(dYb) || !aligned16(work) ||
       !aligned16(grad))

@@ -210,6 +210,8 @@ template <int C>
 struct Cols { // C consecutive BF16 columns of a row
   unsigned d[C / 2];
 };
+// Features may start at any value of their array: a row's 32 go in pairs.
+typedef unsigned pair2u __attribute__((aligned(2)));
 template <int C>
 __device__ inline Cols<C> load_cols(const bf16* p) {
   Cols<C> v;
@@ -224,7 +226,7 @@ __device__ inline Cols<C> load_cols(const bf16* p) {
     v.d[0] = u.x;
     v.d[1] = u.y;
   } else {
-    v.d[0] = *reinterpret_cast<const unsigned*>(p);
+    v.d[0] = *reinterpret_cast<const pair2u*>(p);
   }
   return v;
 }

@@ -88,7 +88,8 @@ int gnn_weight_grad(const gnn_mlp_io* io, const void* G_bf16, const float* G_f32
  *   a residual needs it.  dX[q] = dY costs a launch more; add is none of the dX,
  *   grad = W1 [K][128] | b1 [128] | W2 [128][nout_pad] | b2 [nout_pad].
  * Sources: each 128 wide (gathered or not), or one of 32 without dX; 128
- * outputs, or up to 16 (nout_pad 16, no add).  Arrays 16-byte aligned.
+ * outputs, or up to 16 (nout_pad 16, no add).  Arrays 16-byte aligned, but for
+ * a source of 32 and for dY of up to 16 outputs.
  * work: GNN_GRAD_WORK_FLOATS floats cover every shape.  Deterministic. */
 #define GNN_GRAD_WORK_FLOATS (5L * 1024L * 1024L)
 int gnn_mlp_grads(const gnn_mlp_io* io, const gnn_mlp_weights* w, const float* dY, const float* add,
