@@ -39,9 +39,11 @@ namespace {
 #define DEM_FORCE_MIN_WAVES 1
 #endif
 // Whole passes without bonds or sampling are held to 128 VGPRs (4 waves per
-// SIMD, a few spilled values).  Left alone the compiler takes 150 to 160 (3
-// waves): 4 % slower on the contact-dense bed with the corrected arithmetic,
-// 6 % on the 4M bed with the reference's.  The bonded and sampling variants
+// SIMD).  The reference's lane walk takes 125; the corrected one spills 4 and
+// the tile-spread pass 17 to 34 (36 and 72 to 108 bytes of scratch a lane).
+// Left alone the compiler takes 150 to 160 (3 waves): 4 % slower on the
+// contact-dense bed with the corrected arithmetic, 6 % on the 4M bed with the
+// reference's.  The bonded and sampling variants
 // spill far more at 128 and stay unbounded.
 #ifndef DEM_FORCE_MIN_WAVES_PLAIN
 #define DEM_FORCE_MIN_WAVES_PLAIN 4
@@ -731,6 +733,7 @@ __device__ __forceinline__ void force_tile(const StepArgs& a, const int tile, in
   // requests a wave instead of 80, of 388 requests in all, and the L2 request
   // rate is what the pass runs against (4M spheres, settled: 260 -> 243 us;
   // the same for the loads, whose repeats the L1 absorbs, bought nothing).
+  // Counted since: 88 writes and 159 reads a wave.
   // The bonded kernels would spill for it.
   constexpr bool STAGE = PASS == 0 && KICK != 0 && !BOND;
   const int lane = tid & 63;

@@ -903,8 +903,10 @@ struct NodeFwdArgs {
 #endif
 
 // Where eight waves a CU hold every tile (up to 32,768 nodes on 256 CUs), the
-// pass is one chain per wave: six rows in flight, the mean number of edges a
-// node has, take the aggregation to about one round trip.
+// pass is one chain per wave: six edge rows in flight, about the mean number of
+// edges a node has.  Only whole batches go six at a time; a node's last edges,
+// up to five, come one after the other, and a wave waits for the longest of its
+// 16 nodes.
 constexpr int kNodeSmallWaves = 8, kNodeSmallAgg = 6;
 
 template <int WAVES, int AGG>
