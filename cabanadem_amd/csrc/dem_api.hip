@@ -1568,8 +1568,15 @@ static int graph_cycle(dem_ctx* c) {
     c->rebuilds += 2;
     return DEM_OK;
   }
-  if (c->gexec) { hipGraphExecDestroy(c->gexec); c->gexec = nullptr; }
-  hipError_t e = hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal);
+  hipError_t e = hipSuccess;
+  if (c->gexec) {
+    // the cache decision can change with replays of this graph still queued
+    e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return c->hip_fail(e, "graph sync");
+    hipGraphExecDestroy(c->gexec);
+    c->gexec = nullptr;
+  }
+  e = hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return c->hip_fail(e, "begin capture");
   c->capturing = true;
   int row = 0;
