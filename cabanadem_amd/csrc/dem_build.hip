@@ -502,11 +502,13 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(BuildArgs a) {
 
 // The whole rebuild of a small system in one workgroup: the sequence above with
 // the counts, the sort and the positions in LDS and barriers for launches.  A
-// rebuild of eight launches costs a small system 30 us and more, launch gaps
+// rebuild of seven launches costs a small system 30 us and more, launch gaps
 // for the most part, and by default it comes every step.
 constexpr int kSmallThreads = 1024;
-// Rebuilt every step, us a step with eight launches / one workgroup: 2 spheres
-// 37 / 14, 64 47 / 25, 512 58 / 40, 1,000 60 / 50, 1,728 61 / 78.
+// Rebuilt every step, us a step with the launch sequence / one workgroup: 2
+// spheres 37 / 14, 64 47 / 25, 512 58 / 40, 1,000 60 / 50, 1,728 61 / 78; in
+// coarse binning too (1,000 spheres of 26 neighbours each 154 / 109, of 268
+// 1065 / 560).
 constexpr int kSmallMax = 1024;        // particles
 constexpr int kSmallCells = 8192;      // cells, all systems
 
